@@ -295,40 +295,156 @@ __global__ void sscal_kernel(int n, float alpha, float* x, int incx, grxCycleSlo
   l12_record(probe, t0);
 }
 
-// y = alpha*A*x + beta*y (A m x n col-major): one thread per output row; the
-// column walk keeps lanes on consecutive rows of A, so each step coalesces.
-__global__ void sgemv_n_kernel(int m, int n, float alpha, const float* A, int lda,
-                               const float* x, int incx, float beta, float* y, int incy,
-                               grxCycleSlot* probe) {
+// Four consecutive floats at any 4-byte aligned address: one
+// global_load_dwordx4, which gfx950 takes on dword alignment, so columns of an
+// odd leading dimension are read 16 bytes at a time too.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Element i of a BLAS vector of n elements lies at base + i * inc.
+__device__ __forceinline__ int64_t blas_base(int n, int inc) {
+  return inc > 0 ? 0 : (int64_t)(n - 1) * (-(int64_t)inc);
+}
+
+// y = alpha*A*x + beta*y (A m x n col-major). One workgroup per 4*lr rows:
+// lr lanes cover them, 16 bytes each, and the NT/lr lane groups take every
+// (NT/lr)-th column, U columns' loads in flight per thread; the groups' sums
+// meet in LDS, in a fixed order. No partial result leaves the workgroup, so
+// there is no workspace and no second launch. HBM-bound: 8192 x 4096 26 us,
+// 5.2 TB/s; 16384 x 8192 84 us, 6.4 TB/s (one thread per row, a column per
+// step, was bound by the latency of its one load in flight: 8192 x 4096
+// 970 us). 512 threads with 4 columns in flight were the fastest at every
+// size tried (256 or 1024 threads, 8 or 16 columns: equal to 30 % slower).
+template <int NT, int U>
+__global__ __launch_bounds__(NT) void sgemv_n_kernel(int m, int n, float alpha, const float* A,
+                                                     int lda, const float* x, int incx, float beta,
+                                                     float* y, int incy, int lr,
+                                                     grxCycleSlot* probe) {
   const uint64_t t0 = probe ? cycle_now() : 0;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < m) {
-    float acc = 0.0f;
-    for (int j = 0; j < n; ++j) acc = fmaf(A[(int64_t)j * lda + i], x[blas_index(j, n, incx)], acc);
-    const int64_t yi = blas_index(i, m, incy);
-    y[yi] = (beta == 0.0f) ? alpha * acc : fmaf(beta, y[yi], alpha * acc);
+  __shared__ float part[NT * 4];       // [lane group][row]
+  const int tid = threadIdx.x;
+  // Neighbouring row blocks share cache lines of every column: give each XCD
+  // (workgroups are dealt round-robin over the eight) a contiguous run.
+  const int xcd = blockIdx.x & 7, each = gridDim.x >> 3, more = gridDim.x & 7;
+  const int64_t row0 = (int64_t)(xcd * each + min(xcd, more) + (int)(blockIdx.x >> 3)) * 4 * lr;
+  const int cg = tid / lr, ncg = NT / lr;
+  const int64_t row = row0 + 4 * (tid - cg * lr);
+  const float* a = A + row;
+  const float* xb = x + blas_base(n, incx);
+  const bool full = row + 4 <= m;
+  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (cg < ncg && row < m) {
+    for (int64_t j0 = cg; j0 < n; j0 += U * ncg) {
+      f32x4 av[U];
+      float xv[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        // Columns past n repeat the last one and are dropped below.
+        const int64_t j = min(j0 + u * ncg, (int64_t)n - 1);
+        xv[u] = xb[j * incx];
+        if (full) {
+          av[u] = *(const f32x4u*)(a + j * lda);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) av[u][e] = row + e < m ? a[j * lda + e] : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (j0 + u * ncg < n) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[e] = fmaf(av[u][e], xv[u], acc[e]);
+        }
+    }
+  }
+  *(f32x4*)&part[4 * tid] = acc;       // tid = cg * lr + lane, so rows of a group are adjacent
+  // Halve the groups until one is left: group g takes group g + half.
+  for (int groups = ncg; groups > 1;) {
+    __syncthreads();
+    const int half = (groups + 1) >> 1;
+    if (cg < groups - half) {
+      const f32x4 o = *(const f32x4*)&part[4 * (tid + half * lr)];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] += o[e];
+      *(f32x4*)&part[4 * tid] = acc;
+    }
+    groups = half;
+  }
+  __syncthreads();
+  for (int r = tid; r < 4 * lr; r += NT) {
+    const int64_t i = row0 + r;
+    if (i >= m) break;
+    const float t = part[r];
+    float* yp = y + blas_index((int)i, m, incy);
+    *yp = (beta == 0.0f) ? alpha * t : fmaf(beta, *yp, alpha * t);
   }
   l12_record(probe, t0);
 }
 
-// y = alpha*A^T*x + beta*y: one 256-thread workgroup per output, the lanes
-// stride down a column of A together and reduce in LDS.
+// y = alpha*A^T*x + beta*y: WPC waves of a 256-thread workgroup take NC
+// columns together, striding down them 16 bytes per lane with x read once for
+// all of them; one reduction per column over the lanes, and for WPC = 4 over
+// the waves through LDS in a fixed order. HBM-bound: 8192 x 4096 23.7 us, 5.7
+// TB/s; 1000 x 8191 7.0 us (4-byte loads, a workgroup per column: 26.1 us
+// at 8192 x 4096).
+template <int WPC, int NC>
 __global__ __launch_bounds__(256) void sgemv_t_kernel(int m, int n, float alpha, const float* A,
                                                       int lda, const float* x, int incx, float beta,
                                                       float* y, int incy, grxCycleSlot* probe) {
+  static_assert(WPC == 1 || WPC == 4, "one wave or the whole workgroup per column group");
   const uint64_t t0 = probe ? cycle_now() : 0;
-  __shared__ float part[4];
-  const int j = blockIdx.x;
-  float acc = 0.0f;
-  for (int i = threadIdx.x; i < m; i += 256)
-    acc = fmaf(A[(int64_t)j * lda + i], x[blas_index(i, m, incx)], acc);
-  acc = wave_sum(acc);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const float t = (part[0] + part[1]) + (part[2] + part[3]);
-    const int64_t yi = blas_index(j, n, incy);
-    y[yi] = (beta == 0.0f) ? alpha * t : fmaf(beta, y[yi], alpha * t);
+  __shared__ float part[4][NC];
+  const int wave = threadIdx.x >> 6;
+  const int t = WPC == 4 ? (int)threadIdx.x : (int)threadIdx.x & 63;
+  const int j0 = (WPC == 4 ? (int)blockIdx.x : (int)blockIdx.x * 4 + wave) * NC;
+  const float* xb = x + blas_base(m, incx);
+  float acc[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) acc[c] = 0.0f;
+  const float* a[NC];   // columns past n repeat the last one; their sums are not stored
+#pragma unroll
+  for (int c = 0; c < NC; ++c) a[c] = A + (int64_t)min(j0 + c, n - 1) * lda;
+  const int m4 = m & ~3;
+  constexpr int STEP = 4 * 64 * WPC;
+  auto rows4 = [&](int64_t i) __attribute__((always_inline)) {
+    f32x4 xv, av[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) av[c] = *(const f32x4u*)(a[c] + i);
+    if (incx == 1) {
+      xv = *(const f32x4u*)(xb + i);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) xv[e] = xb[(i + e) * incx];
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[c] = fmaf(av[c][e], xv[e], acc[c]);
+  };
+#pragma unroll 4
+  for (int64_t i = 4 * t; i < m4; i += STEP) rows4(i);
+  if (t < m - m4) {
+    const float xv = xb[(int64_t)(m4 + t) * incx];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[c] = fmaf(a[c][m4 + t], xv, acc[c]);
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c) acc[c] = wave_sum(acc[c]);
+  if (WPC == 4) {
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) part[wave][c] = acc[c];
+    __syncthreads();
+  }
+  if (t < NC && j0 + t < n) {
+    float s = 0.0f;
+    if (WPC == 4) {
+      s = (part[0][t] + part[1][t]) + (part[2][t] + part[3][t]);
+    } else {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) s = c == t ? acc[c] : s;
+    }
+    float* yp = y + blas_index(j0 + t, n, incy);
+    *yp = (beta == 0.0f) ? alpha * s : fmaf(beta, *yp, alpha * s);
   }
   l12_record(probe, t0);
 }
@@ -407,16 +523,39 @@ hipError_t launch_sscal(int n, float alpha, float* x, int incx, grxCycleSlot* pr
   return hipGetLastError();
 }
 
-hipError_t launch_sgemv(bool trans, int m, int n, float alpha, const float* A, int lda,
-                        const float* x, int incx, float beta, float* y, int incy,
-                        grxCycleSlot* probe, hipStream_t s) {
-  const unsigned blocks = (unsigned)sgemv_blocks(trans, m, n);
-  if (!trans) {
-    hipLaunchKernelGGL(sgemv_n_kernel, dim3(blocks), dim3(256), 0, s, m, n, alpha, A, lda, x, incx,
-                       beta, y, incy, probe);
+hipError_t launch_sgemv(bool trans, int m, int n, float alpha, const float* A,
+                        int lda, const float* x, int incx, float beta, float* y,
+                        int incy, grxCycleSlot* probe, hipStream_t s) {
+  // With a cycle probe the launch has the geometry its slots are counted for
+  // (sgemv_blocks): a column per workgroup, or 256 rows.
+  if (trans) {
+    // Two columns per workgroup share each read of x; columns of up to 512
+    // rows fit one wave, which then needs no LDS step (128 x 8192: 2.9
+    // against 4.7 us; 2047 x 2000: 4.7 us with four waves, 5.9 with one).
+    auto go = [&](auto kern, int64_t blocks) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, s, m, n, alpha, A, lda, x, incx,
+                         beta, y, incy, probe);
+    };
+    if (probe) go(sgemv_t_kernel<4, 1>, sgemv_blocks(true, m, n));
+    else if (m <= 512) go(sgemv_t_kernel<1, 2>, ((int64_t)n + 7) / 8);
+    else go(sgemv_t_kernel<4, 2>, ((int64_t)n + 1) / 2);
+    return hipGetLastError();
+  }
+  auto go = [&](auto kern, int threads, int lr) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)(((int64_t)m + 4 * lr - 1) / (4 * lr))), dim3(threads), 0, s,
+                       m, n, alpha, A, lda, x, incx, beta, y, incy, lr, probe);
+  };
+  // Rows per workgroup: as many as leave one workgroup per CU in the fewest
+  // passes over the 256 CUs, since a second workgroup on some CUs doubles the
+  // call (9336 x 4451: 45.8 us as 584 workgroups of 16 rows, 62 as 292 of 32,
+  // 29.4 as 234 of 40). At least 8, so that a wave's 16-byte loads of one
+  // column are 32 bytes together (1000 x 8191: 13.6 us against 14.4 at 4).
+  if (probe) {
+    go(sgemv_n_kernel<256, 8>, 256, 64);
   } else {
-    hipLaunchKernelGGL(sgemv_t_kernel, dim3(blocks), dim3(256), 0, s, m, n, alpha, A, lda, x, incx,
-                       beta, y, incy, probe);
+    const int64_t passes = ((int64_t)m + 16383) / 16384;
+    const int64_t lr = ((int64_t)m + 1024 * passes - 1) / (1024 * passes);
+    go(sgemv_n_kernel<512, 4>, 512, lr < 2 ? 2 : (int)lr);
   }
   return hipGetLastError();
 }

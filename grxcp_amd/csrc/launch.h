@@ -87,7 +87,8 @@ struct SgemmDesc {
 };
 hipError_t launch_sgemm(const SgemmDesc& d, hipStream_t s);
 
-// Level 1/2, fp32 (256-thread workgroups; with a probe, 4 slots per workgroup).
+// Level 1/2, fp32. With a probe the launches are of l1_blocks / sgemv_blocks
+// workgroups of 256 threads, 4 slots each.
 int64_t l1_blocks(int n);
 int64_t sgemv_blocks(bool trans, int m, int n);
 hipError_t launch_saxpy(int n, float alpha, const float* x, int incx, float* y,

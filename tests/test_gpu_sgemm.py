@@ -228,6 +228,28 @@ def test_sscal(blas, n, incx):
 
 
 @pytest.mark.parametrize("trans", [0, 1])
+@pytest.mark.parametrize("m,n", [(1, 1), (3, 700), (8, 1025), (511, 3), (512, 17), (513, 9), (1024, 9), (2049, 130),
+                                 (4100, 257), (16385, 11), (40000, 3)])
+def test_sgemv_workgroup_shapes(blas, trans, m, n):
+    """Row blocks of 8 to 64 rows (one and more passes over the CUs, ragged
+    last blocks), columns in one wave and in four, odd column counts and an
+    odd leading dimension. Whole numbers throughout (every partial sum below
+    2^24), so any order of the sums gives the same bits."""
+    lda = m + 3 - (m & 1)
+    r = np.random.default_rng(m + n)
+    A = r.integers(-3, 4, lda * n).astype(np.float32)
+    xl, yl = (m, n) if trans else (n, m)
+    x, y = (r.integers(-3, 4, k).astype(np.float32) for k in (xl, yl))
+    Am = A.reshape(n, lda)[:, :m].astype(np.float64)
+    want = 2.0 * (Am @ x if trans else x.astype(np.float64) @ Am) + 3.0 * y
+    dA, dx, dy = to_dev(A), to_dev(x), to_dev(y)
+    say(f"sgemv trans={trans} {m}x{n} lda={lda}")
+    assert blas.L.grxblasSgemv(blas.h, trans, m, n, g.fptr(2.0), dA.p, lda, dx.p, 1, g.fptr(3.0), dy.p, 1) == 0
+    g.synchronize()
+    assert np.array_equal(dy.download(np.float32, yl), want.astype(np.float32))
+
+
+@pytest.mark.parametrize("trans", [0, 1])
 @pytest.mark.parametrize("m,n,lda,incx,incy,beta", [(7, 5, 7, 1, 1, 0.0), (33, 17, 40, 2, -1, 2.0),
                                                     (300, 260, 301, -1, 3, 0.0)])
 def test_sgemv(blas, trans, m, n, lda, incx, incy, beta):
