@@ -9,10 +9,11 @@
 //    wavefront, held packed in registers between the statistics pass and the
 //    output pass; both statistics are in-register wave reductions, so there
 //    is no LDS and no barrier and every wave streams independently;
-//  * longer rows (up to 4096 chunks): one row per workgroup of chunks/2
-//    threads (256, 512 or 1024), two chunks per thread held in registers,
-//    one LDS combine per statistic; x is still read from HBM exactly once;
-//  * longer still: x re-read per pass (from L2);
+//  * longer rows (up to 16384 chunks, every length the entry points take):
+//    one row per workgroup of chunks/2 threads (256, 512 or 1024), two
+//    chunks per thread held in registers (four, eight or sixteen past 2048
+//    chunks), one LDS combine per statistic; x is still read from HBM
+//    exactly once;
 //  * 16-byte non-temporal loads of x and stores of y, gamma/beta via the
 //    normal cached path (every row reuses them);
 //  * statistics in fp32: wavefront butterfly (DPP and row swaps) then an LDS
@@ -20,8 +21,9 @@
 //    sees the same value.
 //    LayerNorm's variance is the two-pass (x - mean)^2 form over the cached
 //    registers, which costs no extra memory traffic.
-// Rows whose length, pitch or base alignment rule out 16-byte chunks take a
-// scalar path with the same arithmetic.
+//  * rows whose length, pitch or base alignment rule out 16-byte boundaries
+//    run the same kernels with chunks at element alignment and a partial last
+//    chunk (AL = false).
 
 #include "../launch.h"
 #include "device_common.h"
@@ -29,6 +31,8 @@
 
 namespace grxk {
 namespace {
+
+constexpr u32x4 kZero = {0, 0, 0, 0};
 
 struct NParams {
   const uint8_t* x;
@@ -39,17 +43,9 @@ struct NParams {
   int64_t rows;
   int rows_per_wg;     // norm_block: adjacent rows per workgroup
   int hidden;
+  int align_mask;      // unaligned rows: RowChunks
   float eps;
 };
-
-// Sum over the 256-thread workgroup, identical in every thread.
-__device__ __forceinline__ float block_sum(float v, float* red) {
-  v = wave_sum(v);
-  __syncthreads();  // red[] may still be read from a previous reduction
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return (red[0] + red[1]) + (red[2] + red[3]);
-}
 
 // One row per NT-thread workgroup, NQ 16-byte chunks per thread (chunk
 // tid + NT*q), for rows longer than a wavefront handles well. Measured on
@@ -69,14 +65,13 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 // measured slower. The partials alternate between two LDS slots by row, so
 // a wave still reading one row's partials cannot see the next row's writes,
 // and the loop needs no barrier of its own.
-template <NormType T, bool LAYER, int NT, int NQ>
+template <NormType T, bool AL, bool LAYER, int NT, int NQ>
 __global__ __launch_bounds__(NT) void norm_block(NParams p) {
   using IO = Io<T>;
   constexpr int V = IO::kVec;
   constexpr int NW = NT / 64;
   __shared__ float red[2][2][NW];   // [row parity][statistic][wave]
   const int tid = threadIdx.x;
-  const int nchunks = p.hidden / V;
   const float inv_h = 1.0f / (float)p.hidden;
   int parity = 0;
   auto combine = [&](float v, int slot) {
@@ -88,25 +83,35 @@ __global__ __launch_bounds__(NT) void norm_block(NParams p) {
     for (int w = 0; w < NW; ++w) t += red[parity][slot][w];
     return t;
   };
-  u32x4 graw[NQ], braw[NQ];
+  // gamma and beta are held beside the row (aligned rows: for all rows of
+  // the workgroup; others have their chunks at offsets of their own). With
+  // more than 4 chunks per thread the registers hold the row alone, and gamma
+  // and beta are read when they are used.
+  constexpr bool HOLD = NQ <= 4;
+  u32x4 graw[HOLD ? NQ : 1], braw[HOLD ? NQ : 1];
+  auto weights = [&](const RowChunks<T, AL>& rc) __attribute__((always_inline)) {
+    if constexpr (HOLD)
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const int c = tid + NT * q;
-    graw[q] = c < nchunks ? ((const u32x4*)p.gamma)[c] : u32x4{0, 0, 0, 0};
-    braw[q] = (LAYER && c < nchunks) ? ((const u32x4*)p.beta)[c] : u32x4{0, 0, 0, 0};
-  }
+      for (int q = 0; q < NQ; ++q) {
+        const int c = tid + NT * q;
+        graw[q] = rc.template load<false>(p.gamma, c, kZero);
+        braw[q] = LAYER ? rc.template load<false>(p.beta, c, kZero) : kZero;
+      }
+  };
+  if constexpr (AL) weights(RowChunks<T, AL>(p.x, p.hidden, 0));
 
   const int64_t rb = p.rows_per_wg;
   for (int64_t base = (int64_t)blockIdx.x * rb; base < p.rows; base += (int64_t)gridDim.x * rb)
   for (int64_t row = base, rend = min(p.rows, base + rb); row < rend; ++row, parity ^= 1) {
     const uint8_t* xrow = p.x + row * p.x_rs * (int64_t)(16 / V);
     uint8_t* yrow = p.y + row * p.y_rs * (int64_t)(16 / V);
+    const RowChunks<T, AL> rc(xrow, p.hidden, p.align_mask);
     u32x4 raw[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-      const int c = tid + NT * q;
-      raw[q] = c < nchunks ? __builtin_nontemporal_load((const u32x4*)xrow + c) : u32x4{0, 0, 0, 0};
+      raw[q] = rc.load(xrow, tid + NT * q, kZero);
     }
+    if constexpr (!AL) weights(rc);
     float s = 0.0f;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
@@ -116,22 +121,38 @@ __global__ __launch_bounds__(NT) void norm_block(NParams p) {
       for (int e = 0; e < V; ++e) s += LAYER ? v[e] : v[e] * v[e];
     }
     s = combine(s, 0);
+    // Long rows: only the packed row stays live between the passes.
+    if constexpr (NQ >= 8)
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) asm volatile("" : "+v"(raw[q]));
     float mean = 0.0f, inv;
     if (LAYER) {
       mean = s * inv_h;
       float d2 = 0.0f;
 #pragma unroll
       for (int q = 0; q < NQ; ++q) {
-        if (tid + NT * q >= nchunks) continue;
+        const int c = tid + NT * q;
+        if (!rc.any(c)) continue;
         float v[V];
         IO::unpack(raw[q], v);
+        if (AL || rc.whole(c)) {
 #pragma unroll
-        for (int e = 0; e < V; ++e) {
-          const float d = v[e] - mean;
-          d2 += d * d;
+          for (int e = 0; e < V; ++e) {
+            const float d = v[e] - mean;
+            d2 += d * d;
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < V; ++e) {
+            const float d = rc.has(c, e) ? v[e] - mean : 0.0f;
+            d2 += d * d;
+          }
         }
       }
       d2 = combine(d2, 1);
+      if constexpr (NQ >= 8)
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) asm volatile("" : "+v"(raw[q]));
       inv = 1.0f / sqrtf(d2 * inv_h + p.eps);
     } else {
       inv = 1.0f / sqrtf(s * inv_h + p.eps);
@@ -139,20 +160,20 @@ __global__ __launch_bounds__(NT) void norm_block(NParams p) {
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       const int c = tid + NT * q;
-      if (c >= nchunks) continue;
+      if (!rc.any(c)) continue;
       float v[V], g[V], o[V];
       IO::unpack(raw[q], v);
-      IO::unpack(graw[q], g);
+      IO::unpack(HOLD ? graw[HOLD ? q : 0] : rc.template load<false>(p.gamma, c, kZero), g);
       if (LAYER) {
         float b[V];
-        IO::unpack(braw[q], b);
+        IO::unpack(HOLD ? braw[HOLD ? q : 0] : rc.template load<false>(p.beta, c, kZero), b);
 #pragma unroll
         for (int e = 0; e < V; ++e) o[e] = (v[e] - mean) * inv * g[e] + b[e];
       } else {
 #pragma unroll
         for (int e = 0; e < V; ++e) o[e] = v[e] * inv * g[e];
       }
-      __builtin_nontemporal_store(IO::pack(o), (u32x4*)yrow + c);
+      rc.store(yrow, c, IO::pack(o));
     }
   }
 }
@@ -161,23 +182,22 @@ __global__ __launch_bounds__(NT) void norm_block(NParams p) {
 // the row lives in the wave's registers, both statistics are wave
 // reductions (lane moves only: no LDS, no barrier), so every wave streams
 // independently and a CU keeps ~20 rows of loads in flight.
-template <NormType T, bool LAYER, int NC>
+template <NormType T, bool AL, bool LAYER, int NC>
 __global__ __launch_bounds__(256) void norm_wave(NParams p) {
   using IO = Io<T>;
   constexpr int V = IO::kVec;
   const int lane = threadIdx.x & 63;
-  const int nchunks = p.hidden / V;
   const float inv_h = 1.0f / (float)p.hidden;
   const int64_t nwaves = (int64_t)gridDim.x * 4;
 
   for (int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); row < p.rows; row += nwaves) {
     const uint8_t* xrow = p.x + row * p.x_rs * (int64_t)(16 / V);
     uint8_t* yrow = p.y + row * p.y_rs * (int64_t)(16 / V);
+    const RowChunks<T, AL> rc(xrow, p.hidden, p.align_mask);
     u32x4 raw[NC];
 #pragma unroll
     for (int q = 0; q < NC; ++q) {
-      const int c = lane + 64 * q;
-      raw[q] = c < nchunks ? __builtin_nontemporal_load((const u32x4*)xrow + c) : u32x4{0, 0, 0, 0};
+      raw[q] = rc.load(xrow, lane + 64 * q, kZero);
     }
     float s = 0.0f;
 #pragma unroll
@@ -198,13 +218,22 @@ __global__ __launch_bounds__(256) void norm_wave(NParams p) {
       float d2 = 0.0f;
 #pragma unroll
       for (int q = 0; q < NC; ++q) {
-        if (lane + 64 * q >= nchunks) continue;
+        const int c = lane + 64 * q;
+        if (!rc.any(c)) continue;
         float v[V];
         IO::unpack(raw[q], v);
+        if (AL || rc.whole(c)) {
 #pragma unroll
-        for (int e = 0; e < V; ++e) {
-          const float d = v[e] - mean;
-          d2 += d * d;
+          for (int e = 0; e < V; ++e) {
+            const float d = v[e] - mean;
+            d2 += d * d;
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < V; ++e) {
+            const float d = rc.has(c, e) ? v[e] - mean : 0.0f;
+            d2 += d * d;
+          }
         }
       }
       d2 = wave_sum(d2);
@@ -217,59 +246,56 @@ __global__ __launch_bounds__(256) void norm_wave(NParams p) {
 #pragma unroll
     for (int q = 0; q < NC; ++q) {
       const int c = lane + 64 * q;
-      if (c >= nchunks) continue;
+      if (!rc.any(c)) continue;
       float v[V], g[V], o[V];
       IO::unpack(raw[q], v);
-      IO::unpack(((const u32x4*)p.gamma)[c], g);
+      IO::unpack(rc.template load<false>(p.gamma, c, kZero), g);
       if (LAYER) {
         float b[V];
-        IO::unpack(((const u32x4*)p.beta)[c], b);
+        IO::unpack(rc.template load<false>(p.beta, c, kZero), b);
 #pragma unroll
         for (int e = 0; e < V; ++e) o[e] = (v[e] - mean) * inv * g[e] + b[e];
       } else {
 #pragma unroll
         for (int e = 0; e < V; ++e) o[e] = v[e] * inv * g[e];
       }
-      __builtin_nontemporal_store(IO::pack(o), (u32x4*)yrow + c);
+      rc.store(yrow, c, IO::pack(o));
     }
   }
 }
 
-// Any length / alignment: element-wise, x re-read for each pass.
-template <NormType T, bool LAYER>
-__global__ __launch_bounds__(256) void norm_scalar(NParams p) {
-  using IO = Io<T>;
-  __shared__ float red[4];
-  const int tid = threadIdx.x;
-  const float inv_h = 1.0f / (float)p.hidden;
-  for (int64_t row = blockIdx.x; row < p.rows; row += gridDim.x) {
-    const int64_t xo = row * p.x_rs, yo = row * p.y_rs;
-    float s = 0.0f;
-    for (int c = tid; c < p.hidden; c += 256) {
-      const float x = IO::ld(p.x, xo + c);
-      s += LAYER ? x : x * x;
-    }
-    s = block_sum(s, red);
-    float mean = 0.0f, inv;
-    if (LAYER) {
-      mean = s * inv_h;
-      float d2 = 0.0f;
-      for (int c = tid; c < p.hidden; c += 256) {
-        const float d = IO::ld(p.x, xo + c) - mean;
-        d2 += d * d;
-      }
-      d2 = block_sum(d2, red);
-      inv = 1.0f / sqrtf(d2 * inv_h + p.eps);
-    } else {
-      inv = 1.0f / sqrtf(s * inv_h + p.eps);
-    }
-    for (int c = tid; c < p.hidden; c += 256) {
-      const float x = IO::ld(p.x, xo + c);
-      const float g = IO::ld(p.gamma, c);
-      const float o = LAYER ? (x - mean) * inv * g + IO::ld(p.beta, c) : x * inv * g;
-      IO::st(p.y, yo + c, o);
-    }
-  }
+template <NormType T, bool AL, bool LAYER>
+hipError_t run_rows(NParams p, hipStream_t s) {
+  constexpr int V = Io<T>::kVec;
+  const int nchunks = (p.hidden + V - 1) / V;   // at most 65536 / V (the entry points' limit)
+  if (p.hidden > 65536) return hipErrorNotSupported;
+  const unsigned wgrid = (unsigned)std::min<int64_t>((p.rows + 3) / 4, 1 << 30);
+  // norm_block: two adjacent rows per workgroup where that still leaves at
+  // least four workgroups per CU
+  p.rows_per_wg = p.rows >= 2048 ? 2 : 1;
+  const unsigned bgrid =
+      (unsigned)std::min<int64_t>((p.rows + p.rows_per_wg - 1) / p.rows_per_wg, 1 << 30);
+  // Past 2048 chunks aligned rows run fastest on 1024 threads, others on 512
+  // with twice the chunks (RMSNorm 4096 x 32000 bf16 92 us against 102;
+  // LayerNorm 4096 x 32001 128 against 151). Element-wise passes re-reading
+  // x, which such rows took before: 2 x 45008 73 us, now 7.
+  // cap: chunks the kernel holds. A row off its boundaries takes one chunk
+  // more (its first and last are partial) where a kernel has room for it.
+  const int need = nchunks + (AL ? 0 : 1);
+  auto go = [&](auto kern, int cap, unsigned grid, int threads) {
+    p.align_mask = need <= cap ? V - 1 : 0;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), 0, s, p);
+  };
+  if (need <= 64) go(norm_wave<T, AL, LAYER, 1>, 64, wgrid, 256);
+  else if (need <= 128) go(norm_wave<T, AL, LAYER, 2>, 128, wgrid, 256);
+  else if (need <= 256) go(norm_wave<T, AL, LAYER, 4>, 256, wgrid, 256);
+  else if (need <= 512) go(norm_block<T, AL, LAYER, 256, 2>, 512, bgrid, 256);
+  else if (need <= 1024) go(norm_block<T, AL, LAYER, 512, 2>, 1024, bgrid, 512);
+  else if (need <= 2048) go(norm_block<T, AL, LAYER, 1024, 2>, 2048, bgrid, 1024);
+  else if (need <= 4096) go(norm_block<T, AL, LAYER, AL ? 1024 : 512, AL ? 4 : 8>, 4096, bgrid, AL ? 1024 : 512);
+  else if (V == 8 || need <= 8192) go(norm_block<T, AL, LAYER, 1024, 8>, 8192, bgrid, 1024);
+  else if constexpr (V == 4) go(norm_block<T, AL, LAYER, 1024, 16>, 16384, bgrid, 1024);
+  return hipGetLastError();
 }
 
 template <NormType T, bool LAYER>
@@ -285,35 +311,10 @@ hipError_t run(const NormDesc& d, hipStream_t s) {
   p.hidden = d.hidden;
   p.eps = d.eps;
   constexpr int V = Io<T>::kVec;
-  const unsigned grid = (unsigned)std::min<int64_t>(d.rows, 1 << 30);
   auto al = [](const void* q) { return ((uintptr_t)q % 16) == 0; };
   const bool vec = d.hidden % V == 0 && d.x_row_stride % V == 0 && d.y_row_stride % V == 0 &&
                    al(d.x) && al(d.y) && al(d.gamma) && (!LAYER || al(d.beta));
-  const int nchunks = d.hidden / V;
-  const unsigned wgrid = (unsigned)std::min<int64_t>((d.rows + 3) / 4, 1 << 30);
-  // norm_block: two adjacent rows per workgroup where that still leaves at
-  // least four workgroups per CU
-  p.rows_per_wg = d.rows >= 2048 ? 2 : 1;
-  const unsigned bgrid =
-      (unsigned)std::min<int64_t>((d.rows + p.rows_per_wg - 1) / p.rows_per_wg, 1 << 30);
-  if (vec && nchunks <= 64) {
-    hipLaunchKernelGGL((norm_wave<T, LAYER, 1>), dim3(wgrid), dim3(256), 0, s, p);
-  } else if (vec && nchunks <= 128) {
-    hipLaunchKernelGGL((norm_wave<T, LAYER, 2>), dim3(wgrid), dim3(256), 0, s, p);
-  } else if (vec && nchunks <= 256) {
-    hipLaunchKernelGGL((norm_wave<T, LAYER, 4>), dim3(wgrid), dim3(256), 0, s, p);
-  } else if (vec && nchunks <= 512) {
-    hipLaunchKernelGGL((norm_block<T, LAYER, 256, 2>), dim3(bgrid), dim3(256), 0, s, p);
-  } else if (vec && nchunks <= 1024) {
-    hipLaunchKernelGGL((norm_block<T, LAYER, 512, 2>), dim3(bgrid), dim3(512), 0, s, p);
-  } else if (vec && nchunks <= 2048) {
-    hipLaunchKernelGGL((norm_block<T, LAYER, 1024, 2>), dim3(bgrid), dim3(1024), 0, s, p);
-  } else if (vec && nchunks <= 4096) {
-    hipLaunchKernelGGL((norm_block<T, LAYER, 1024, 4>), dim3(bgrid), dim3(1024), 0, s, p);
-  } else {
-    hipLaunchKernelGGL((norm_scalar<T, LAYER>), dim3(grid), dim3(256), 0, s, p);
-  }
-  return hipGetLastError();
+  return vec ? run_rows<T, true, LAYER>(p, s) : run_rows<T, false, LAYER>(p, s);
 }
 
 }  // namespace
