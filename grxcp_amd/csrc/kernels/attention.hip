@@ -42,10 +42,15 @@
 //    (all query tiles of a head on one XCD: K/V shared in its L2), each
 //    XCD's items are dealt a block of heads at a time, heaviest first, in a
 //    snake order, so every CU gets the same number of key tiles (272 of
-//    69632 at B4 H32 S4096) and an XCD's CUs share few heads' K/V at a time.
+//    69632 at B4 H32 S4096) and an XCD's CUs share few heads' K/V at a time;
+//  * problems whose 256-query items would leave CUs idle take attn_split:
+//    items of 128 or 64 queries, a workgroup's waves split over the keys.
 
 #include "../launch.h"
 #include "device_common.h"
+
+#include <algorithm>
+#include <cmath>
 
 namespace grxk {
 namespace {
@@ -145,6 +150,7 @@ struct AParams {
   int B, H, S;
   int qtiles;
   int heads;      // B * H
+  int hb;         // heads per block of an XCD's items (attn_fwd)
   int causal;
   float c;  // scale * log2(e)
   grxCycleSlot* probe;   // one slot per wave, or null
@@ -184,7 +190,8 @@ __device__ __forceinline__ float half_swap_sum(float x) {
 // and right to left for odd r: two rounds give every workgroup the same
 // number of key tiles, and the workgroups of an XCD share few heads' K/V at
 // a time (B4 H32 S4096: FETCH_SIZE 564 MB per launch, against 1420 MB when
-// a round took the heaviest tiles of all 16 heads of the XCD).
+// a round took the heaviest tiles of all 16 heads of the XCD). Where a few
+// rounds do not come out even that way, all heads are one block (heads_per_block).
 struct ItemMap {
   int xcd, wg, nwg;     // this workgroup's XCD, index within it, workgroups per XCD
   int hx;               // heads on this XCD
@@ -195,9 +202,7 @@ __device__ __forceinline__ bool item_at(const AParams& p, const ItemMap& m, int 
   const int k = (round & 1) ? (m.nwg - 1 - m.wg) : m.wg;
   const int j = round * m.nwg + k;
   if (j >= nloc || m.hx == 0) return false;
-  int hb = m.nwg / p.qtiles;          // heads per block
-  if (hb < 1) hb = 1;
-  if (hb > m.hx) hb = m.hx;
+  const int hb = min(p.hb, m.hx);     // heads per block
   const int blk_items = hb * p.qtiles;
   const int blk = j / blk_items;
   const int r2 = j - blk * blk_items;
@@ -207,6 +212,127 @@ __device__ __forceinline__ bool item_at(const AParams& p, const ItemMap& m, int 
   *bh = m.xcd + 8 * hl;
   *qt = p.causal ? (p.qtiles - 1 - rank) : rank;
   return true;
+}
+
+// A lane's place in the fragments: query (and key row) l32, half hh, and the
+// key and head-dim offsets of its transposing V reads.
+struct LanePos {
+  int l32, hh, tr_key, tr_d;
+};
+__device__ __forceinline__ LanePos lane_pos(int lane) {
+  LanePos l;
+  l.l32 = lane & 31;
+  l.hh = lane >> 5;
+  l.tr_key = 4 * l.hh + ((lane & 15) >> 2);
+  l.tr_d = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  return l;
+}
+
+// One 64-key tile (keys kv0 .. kv0+63; K rows at kt, V rows at vt in LDS) for
+// the wave's queries wq0 .. wq0+31: scores, online softmax, O^T += V^T P^T.
+template <AttnType T, int D>
+__device__ __forceinline__ void attend_tile(const AParams& p, const LanePos& l, const i32x4* kt,
+                                            const uint8_t* vt, int kv0, int wq0,
+                                            const i32x4 (&qf)[D / 16], f32x16 (&o_acc)[D / 32],
+                                            float& m_run, float& l_run) {
+  using IO = AIo<T>;
+  constexpr int CH = D / 8, DSTEPS = D / 16, DT = D / 32;
+    // S^T for keys 0-31 and 32-63: two independent accumulation chains,
+    // issued alternately, with the K fragments read kQkAhead MFMAs ahead
+    // of their use (the schedule is pinned below: left to itself the
+    // compiler reads each fragment just before its MFMA and waits for it,
+    // 4-5 % slower).
+    f32x16 s[2];
+    {
+      i32x4 kf[DSTEPS][2];
+#pragma unroll
+      for (int d = 0; d < DSTEPS; ++d)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+          const int row = kb * 32 + l.l32;
+          kf[d][kb] = kt[row * CH + ((2 * d + l.hh) ^ kswz<D>(row))];
+        }
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[kb][r] = 0.0f;
+#pragma unroll
+      for (int d = 0; d < DSTEPS; ++d)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) s[kb] = IO::mma(kf[d][kb], qf[d], s[kb]);
+    }
+    // instruction groups, in order: kQkAhead LDS reads, then alternately
+    // one MFMA and one read, then the last kQkAhead MFMAs
+    __builtin_amdgcn_sched_group_barrier(0x100, kQkAhead, 0);
+#pragma unroll
+    for (int i = 0; i < 2 * DSTEPS - kQkAhead; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, kQkAhead, 0);
+    const bool need_mask = (kv0 + kBK > p.S) || (p.causal && kv0 + kBK - 1 > wq0);
+    if (need_mask) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int key = kv0 + kb * 32 + 8 * (r >> 2) + 4 * l.hh + (r & 3);
+          const bool masked = key >= p.S || (p.causal && key > wq0 + l.l32);
+          s[kb][r] = masked ? -INFINITY : s[kb][r];
+        }
+    }
+    uint32_t pk[2][8];
+    {
+      float mx0 = -INFINITY, mx1 = -INFINITY;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        mx0 = fmaxf(mx0, s[0][r]);
+        mx1 = fmaxf(mx1, s[1][r]);
+      }
+      const float mx = half_swap_max(fmaxf(mx0, mx1)) * p.c;
+      const bool raise = mx > m_run + 8.0f;
+      if (__builtin_amdgcn_ballot_w64(raise)) {
+        const float m_new = raise ? mx : m_run;
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        m_run = m_new;
+        l_run *= alpha;
+#pragma unroll
+        for (int i = 0; i < DT; ++i)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o_acc[i][r] *= alpha;
+      }
+      const float m = m_run;
+      float ps0 = 0.0f, ps1 = 0.0f;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+          const float p0 = __builtin_amdgcn_exp2f(fmaf(s[kb][r], p.c, -m));
+          const float p1 = __builtin_amdgcn_exp2f(fmaf(s[kb][r + 1], p.c, -m));
+          pk[kb][r >> 1] = IO::pack2(p0, p1);
+          if (kb == 0) ps0 = IO::sum2(pk[kb][r >> 1], ps0);
+          else ps1 = IO::sum2(pk[kb][r >> 1], ps1);
+        }
+      l_run += ps0 + ps1;
+    }
+#pragma unroll
+    for (int st = 0; st < kBK / 16; ++st) {
+      const int kb = st >> 1, half = st & 1;
+      const i32x4 pf4 = i32x4{(int)pk[kb][4 * half + 0], (int)pk[kb][4 * half + 1],
+                              (int)pk[kb][4 * half + 2], (int)pk[kb][4 * half + 3]};
+      const int k1 = 16 * st + l.tr_key, k2 = k1 + 8;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const int d = 32 * dt + l.tr_d;
+        const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_s16x4_t)(vt + k1 * (2 * D) + 16 * ((d >> 3) ^ vswz<D>(k1)) + 2 * (d & 7)));
+        const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_s16x4_t)(vt + k2 * (2 * D) + 16 * ((d >> 3) ^ vswz<D>(k2)) + 2 * (d & 7)));
+        const u32x2 w0 = __builtin_bit_cast(u32x2, v0), w1 = __builtin_bit_cast(u32x2, v1);
+        const i32x4 vf = i32x4{(int)w0.x, (int)w0.y, (int)w1.x, (int)w1.y};
+        o_acc[dt] = IO::mma(vf, pf4, o_acc[dt]);
+      }
+    }
 }
 
 template <AttnType T, int D>
@@ -339,8 +465,7 @@ __global__ __launch_bounds__(64 * kNW, 1) void attn_fwd(AParams p) {
   float m_run = -INFINITY;
   float l_run = 0.0f;
 
-  const int tr_key = 4 * hh + ((lane & 15) >> 2);
-  const int tr_d = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  const LanePos lp = lane_pos(lane);
 
   int t = 0;          // tile of the current item
   bool done = false;
@@ -357,107 +482,11 @@ __global__ __launch_bounds__(64 * kNW, 1) void attn_fwd(AParams p) {
     }
     const int kv0 = t * kBK;
     const int wq0 = cur.q0 + 32 * wave;
-    const int myq = wq0 + l32;
     const i32x4* kt = &lds[cs][0][0];
     const uint8_t* vt = (const uint8_t*)&lds[cs][1][0];
     const bool wave_live = !p.causal || kv0 <= wq0 + 31;
     if (wave_live) {
-      // S^T for keys 0-31 and 32-63: two independent accumulation chains,
-      // issued alternately, with the K fragments read kQkAhead MFMAs ahead
-      // of their use (the schedule is pinned below: left to itself the
-      // compiler reads each fragment just before its MFMA and waits for it,
-      // 4-5 % slower).
-      f32x16 s[2];
-      {
-        i32x4 kf[DSTEPS][2];
-#pragma unroll
-        for (int d = 0; d < DSTEPS; ++d)
-#pragma unroll
-          for (int kb = 0; kb < 2; ++kb) {
-            const int row = kb * 32 + l32;
-            kf[d][kb] = kt[row * CH + ((2 * d + hh) ^ kswz<D>(row))];
-          }
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) s[kb][r] = 0.0f;
-#pragma unroll
-        for (int d = 0; d < DSTEPS; ++d)
-#pragma unroll
-          for (int kb = 0; kb < 2; ++kb) s[kb] = IO::mma(kf[d][kb], qf[d], s[kb]);
-      }
-      // instruction groups, in order: kQkAhead LDS reads, then alternately
-      // one MFMA and one read, then the last kQkAhead MFMAs
-      __builtin_amdgcn_sched_group_barrier(0x100, kQkAhead, 0);
-#pragma unroll
-      for (int i = 0; i < 2 * DSTEPS - kQkAhead; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      }
-      __builtin_amdgcn_sched_group_barrier(0x008, kQkAhead, 0);
-      const bool need_mask = (kv0 + kBK > p.S) || (p.causal && kv0 + kBK - 1 > wq0);
-      if (need_mask) {
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = kv0 + kb * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
-            const bool masked = key >= p.S || (p.causal && key > myq);
-            s[kb][r] = masked ? -INFINITY : s[kb][r];
-          }
-      }
-      uint32_t pk[2][8];
-      {
-        float mx0 = -INFINITY, mx1 = -INFINITY;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          mx0 = fmaxf(mx0, s[0][r]);
-          mx1 = fmaxf(mx1, s[1][r]);
-        }
-        const float mx = half_swap_max(fmaxf(mx0, mx1)) * p.c;
-        const bool raise = mx > m_run + 8.0f;
-        if (__builtin_amdgcn_ballot_w64(raise)) {
-          const float m_new = raise ? mx : m_run;
-          const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-          m_run = m_new;
-          l_run *= alpha;
-#pragma unroll
-          for (int i = 0; i < DT; ++i)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) o_acc[i][r] *= alpha;
-        }
-        const float m = m_run;
-        float ps0 = 0.0f, ps1 = 0.0f;
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int r = 0; r < 16; r += 2) {
-            const float p0 = __builtin_amdgcn_exp2f(fmaf(s[kb][r], p.c, -m));
-            const float p1 = __builtin_amdgcn_exp2f(fmaf(s[kb][r + 1], p.c, -m));
-            pk[kb][r >> 1] = IO::pack2(p0, p1);
-            if (kb == 0) ps0 = IO::sum2(pk[kb][r >> 1], ps0);
-            else ps1 = IO::sum2(pk[kb][r >> 1], ps1);
-          }
-        l_run += ps0 + ps1;
-      }
-#pragma unroll
-      for (int st = 0; st < kBK / 16; ++st) {
-        const int kb = st >> 1, half = st & 1;
-        const i32x4 pf4 = i32x4{(int)pk[kb][4 * half + 0], (int)pk[kb][4 * half + 1],
-                                (int)pk[kb][4 * half + 2], (int)pk[kb][4 * half + 3]};
-        const int k1 = 16 * st + tr_key, k2 = k1 + 8;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          const int d = 32 * dt + tr_d;
-          const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (lds_s16x4_t)(vt + k1 * (2 * D) + 16 * ((d >> 3) ^ vswz<D>(k1)) + 2 * (d & 7)));
-          const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (lds_s16x4_t)(vt + k2 * (2 * D) + 16 * ((d >> 3) ^ vswz<D>(k2)) + 2 * (d & 7)));
-          const u32x2 w0 = __builtin_bit_cast(u32x2, v0), w1 = __builtin_bit_cast(u32x2, v1);
-          const i32x4 vf = i32x4{(int)w0.x, (int)w0.y, (int)w1.x, (int)w1.y};
-          o_acc[dt] = IO::mma(vf, pf4, o_acc[dt]);
-        }
-      }
+      attend_tile<T, D>(p, lp, kt, vt, kv0, wq0, qf, o_acc, m_run, l_run);
     }
     if (last) {
       // O[q, d] = O^T[d, q] / l for this item; then start the next one.
@@ -531,6 +560,167 @@ __global__ __launch_bounds__(64 * kNW, 1) void attn_fwd(AParams p) {
   cycle_record(p.probe, t_start, blockIdx.x * kNW + wave, wave);
 }
 
+// Problems of few query tiles: one workgroup per item of 32*QW queries of one
+// head, whose 8 waves are QW query blocks of 32 times KS = 8/QW key groups.
+// Group g takes the 64-key tiles g, g + KS, ..., with the running maximum, sum
+// and O of its own, and the groups' results meet in LDS at the end (O scaled
+// by exp2(m_g - max m), fp32). So a head of S keys takes S/(64*KS) steps on
+// ceil(S/(32*QW)) CUs instead of S/64 on ceil(S/256). NS LDS stages of KS
+// tiles: with two, a step's loads are issued one step ahead; with one (the
+// tiles of a step fill LDS) the next step's loads wait for this one's reads.
+// A wave alone in its group (QW = 1) reads only what it loaded and needs no
+// barrier.
+template <AttnType T, int D, int QW, int NS>
+__global__ __launch_bounds__(64 * kNW, 1) void attn_split(AParams p) {
+  using IO = AIo<T>;
+  constexpr int KS = kNW / QW;
+  constexpr int CH = D / 8, RPI = 64 / CH, DSTEPS = D / 16, DT = D / 32;
+  constexpr int IPW = CH / QW;                     // 1 KB loads per wave, operand and tile
+  constexpr int kTile = kBK * CH;                  // 16-byte chunks of one operand's tile
+  constexpr int kPitch = D + 4;                    // floats per row of a wave's O in LDS
+  constexpr int kStageBytes = NS * KS * 2 * kTile * 16;
+  constexpr int kMergeBytes = kNW * 32 * kPitch * 4;
+  static_assert(NS == 1 || NS == 2, "stages");
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kStageBytes > kMergeBytes ? kStageBytes : kMergeBytes];
+  __shared__ float ml[kNW][2][32];                 // running maximum and sum per query
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = wave / QW, qw = wave % QW;
+  const LanePos lp = lane_pos(lane);
+
+  // Items by weight (causal: the last query tiles first), heads inside: with
+  // heads a multiple of 8 every item of a head runs on one XCD (workgroups are
+  // dealt round-robin over the eight) and its K and V stay in that L2.
+  const int r0 = blockIdx.x / p.heads, bh = blockIdx.x - r0 * p.heads;
+  const int q0 = (p.causal ? p.qtiles - 1 - r0 : r0) * 32 * QW;
+  const int b = bh / p.H, h = bh - b * p.H;
+  const uint32_t q_rs = (uint32_t)(2 * p.q_ss), k_rs = (uint32_t)(2 * p.k_ss), v_rs = (uint32_t)(2 * p.v_ss);
+  const uint32_t o_rs = (uint32_t)(2 * p.o_ss);
+  const i32x4 rk = rsrc_words(p.k + 2 * (b * p.k_sb + h * p.k_sh), (uint32_t)(p.S - 1) * k_rs + 2 * D);
+  const i32x4 rv = rsrc_words(p.v + 2 * (b * p.v_sb + h * p.v_sh), (uint32_t)(p.S - 1) * v_rs + 2 * D);
+  const int kv_end = p.causal ? min(p.S, q0 + 32 * QW) : p.S;
+  const int ntiles = (kv_end + kBK - 1) / kBK;
+  const int steps = (ntiles + KS - 1) / KS;
+
+  uint32_t kbase[IPW], vbase[IPW];
+#pragma unroll
+  for (int i = 0; i < IPW; ++i) {
+    const int row = RPI * (QW * i + qw) + lane / CH;
+    const int pc = lane % CH;
+    kbase[i] = (uint32_t)row * k_rs + (uint32_t)(16 * (pc ^ kswz<D>(row)));
+    vbase[i] = (uint32_t)row * v_rs + (uint32_t)(16 * (pc ^ vswz<D>(row)));
+  }
+  auto tile_at = [&](int st, int operand) { return smem + (((st * KS + g) * 2 + operand) * kTile) * 16; };
+  // The group's tile of step s into stage st.
+  auto load = [&](int s, int st) __attribute__((always_inline)) {
+    const int kv0 = (s * KS + g) * kBK;
+    if (kv0 >= kv_end) return;
+    const bool inside = kv0 + kBK <= p.S;          // rows past S read as zero
+#pragma unroll
+    for (int i = 0; i < IPW; ++i) {
+      const uint32_t lk = lds_addr(tile_at(st, 0) + 1024 * (QW * i + qw));
+      const uint32_t lv = lds_addr(tile_at(st, 1) + 1024 * (QW * i + qw));
+      if (inside) {
+        dma16_so(rk, lk, kbase[i], (uint32_t)kv0 * k_rs);
+        dma16_so(rv, lv, vbase[i], (uint32_t)kv0 * v_rs);
+      } else {
+        dma16(rk, lk, (uint32_t)kv0 * k_rs + kbase[i]);
+        dma16(rv, lv, (uint32_t)kv0 * v_rs + vbase[i]);
+      }
+    }
+  };
+  auto landed = [&]() __attribute__((always_inline)) {
+    wait_vmem_all();
+    if constexpr (QW > 1) __syncthreads();
+  };
+
+  load(0, 0);
+  const int wq0 = q0 + 32 * qw;
+  i32x4 qf[DSTEPS];
+  {
+    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(p.q + 2 * (b * p.q_sb + h * p.q_sh)), (short)0, (int)((uint32_t)(p.S - 1) * q_rs + 2 * D),
+        kRsrcWord3);
+#pragma unroll
+    for (int t = 0; t < DSTEPS; ++t)
+      qf[t] = __builtin_amdgcn_raw_buffer_load_b128(
+          rq, (uint32_t)(wq0 + lp.l32) * q_rs + (uint32_t)(2 * (16 * t + 8 * lp.hh)), 0, 0);
+  }
+  f32x16 o_acc[DT];
+#pragma unroll
+  for (int i = 0; i < DT; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o_acc[i][r] = 0.0f;
+  float m_run = -INFINITY, l_run = 0.0f;
+  landed();
+  for (int s = 0; s < steps; ++s) {
+    const int st = NS == 2 ? s & 1 : 0;
+    if (NS == 2 && s + 1 < steps) load(s + 1, st ^ 1);
+    const int kv0 = (s * KS + g) * kBK;
+    if (kv0 < kv_end && (!p.causal || kv0 <= wq0 + 31))
+      attend_tile<T, D>(p, lp, (const i32x4*)tile_at(st, 0), tile_at(st, 1), kv0, wq0, qf, o_acc, m_run, l_run);
+    if (NS == 1 && s + 1 < steps) {
+      // every read of this step's tiles is done before the next one's land
+      if constexpr (QW > 1) __syncthreads();
+      else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      load(s + 1, 0);
+    }
+    if (s + 1 < steps) landed();
+  }
+
+  // The groups' O, maximum and sum to LDS, over the tiles.
+  const float l_tot = half_swap_sum(l_run);
+  __syncthreads();
+  float* mo = (float*)smem;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const f32x4 v = {o_acc[dt][4 * r], o_acc[dt][4 * r + 1], o_acc[dt][4 * r + 2], o_acc[dt][4 * r + 3]};
+      *(f32x4*)&mo[(wave * 32 + lp.l32) * kPitch + 32 * dt + 8 * r + 4 * lp.hh] = v;
+    }
+  if (lp.hh == 0) {
+    ml[wave][0][lp.l32] = m_run;
+    ml[wave][1][lp.l32] = l_tot;
+  }
+  __syncthreads();
+  // Wave (g, qw) combines rows g*32/KS .. of query block qw, 8 values per lane.
+  constexpr int ROWS = 32 / KS;
+  const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(p.o + 2 * (b * p.o_sb + h * p.o_sh)), (short)0, (int)((uint32_t)(p.S - 1) * o_rs + 2 * D), kRsrcWord3);
+  const int cc = lane % CH;
+  for (int rr = lane / CH; rr < ROWS; rr += RPI) {
+    const int row = g * ROWS + rr;
+    float mx = ml[qw][0][row];
+#pragma unroll
+    for (int j = 1; j < KS; ++j) mx = fmaxf(mx, ml[j * QW + qw][0][row]);
+    float l = 0.0f, o[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < KS; ++j) {
+      const int w = j * QW + qw;
+      const float scale = __builtin_amdgcn_exp2f(ml[w][0][row] - mx);
+      l = fmaf(scale, ml[w][1][row], l);
+      const f32x4* src = (const f32x4*)&mo[(w * 32 + row) * kPitch + 8 * cc];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const f32x4 v = src[q];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[4 * q + e] = fmaf(scale, v[e], o[4 * q + e]);
+      }
+    }
+    const float inv_l = l > 0.0f ? 1.0f / l : 0.0f;
+    i32x4 out;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) out[q] = (int)IO::pack2(o[2 * q] * inv_l, o[2 * q + 1] * inv_l);
+    // rows at or past S lie outside the descriptor's range: dropped
+    __builtin_amdgcn_raw_buffer_store_b128(out, ro, (uint32_t)(q0 + 32 * qw + row) * o_rs + 16 * cc, 0, 0);
+  }
+}
+
 // One workgroup per CU, a multiple of 8 (one share per XCD), no more than
 // the items need.
 int64_t workgroups(int B, int H, int S) {
@@ -543,6 +733,58 @@ int64_t workgroups(int B, int H, int S) {
   if (wgs / 8 > per_xcd_items) wgs = 8 * per_xcd_items;
   if (wgs < 8) wgs = 8;
   return wgs;
+}
+
+// Heads per block of attn_fwd's item order: as many as one round of an XCD's
+// workgroups has room for. Causal launches of at most 8 rounds whose rounds do
+// not come out even (a block that is no whole share of a round, a last round
+// that is odd or part empty) would leave a workgroup with two of the heaviest
+// items: their heads are one block, whose snake pairs heavy with light (B2 H20
+// S2500 D64 91 us in blocks of 3 heads).
+int heads_per_block(int64_t hx, int qtiles, int nwg, bool causal) {
+  const int hb = (int)std::max<int64_t>(1, std::min<int64_t>(nwg / qtiles, hx));
+  const int64_t items = hx * qtiles;
+  const bool even = nwg % (hb * qtiles) == 0 && items % (2 * nwg) == 0;
+  return causal && !even && items > nwg && items <= 8 * nwg ? (int)hx : hb;
+}
+
+// Query blocks per workgroup of attn_split (4 or 2), or 0 for the persistent
+// attn_fwd, whichever is modelled fastest (us; the constants fit bf16 times of
+// 64 to 4000 keys on 4 to 256 heads). A CU runs one tile (or step of KS tiles)
+// at a time, so a launch takes the steps of its busiest CU: the heaviest item
+// while there are at most 256, the average CU's share beyond, plus a start and
+// an end per item, which the persistent kernel hides. us, attn_fwd / QW 4 / QW
+// 2: B2 H16 S1000 D64 24.0 / 16.9 / 21.9; B1 H8 S2048 D64 38.6 / 24.0 / 16.5
+// and D128 49.9 / 33.6 / 27.0; B1 H24 S218 D128 12.3 / 9.8 / 8.5; B4 H16
+// S1024 D64 23.5 / 24.1 / 36.2 and D128 36.5 / 43.1 / 63.6.
+int split_blocks(int64_t heads, int S, int D, bool causal) {
+  const double start = D == 64 ? 3.5 : 4.0;
+  // Mean tiles of an item of `queries` over the heaviest item's.
+  auto share = [&](int queries) {
+    const int n = (S + queries - 1) / queries;
+    return causal ? (n + 1.0) / (2.0 * n) : 1.0;
+  };
+  const double tiles = (S + kBK - 1) / kBK;
+  // attn_fwd: the items of one XCD's heads over its 32 workgroups
+  const double items8 = (double)((heads + 7) / 8) * ((S + kBQ - 1) / kBQ) / 32.0;
+  const double rounds = causal ? std::max(1.0, 1.1 * items8 * share(kBQ)) : std::ceil(items8);
+  double best = 0.95 * (start + (D == 64 ? 1.25 : 1.8) * tiles * rounds);
+  int qw = 0;
+  for (int w = 4; w >= 2; w /= 2) {
+    const double items = (double)heads * ((S + 32 * w - 1) / (32 * w)) / 256.0;   // per CU
+    const double steps = std::ceil(tiles * w / kNW) * (items > 1.0 ? share(32 * w) : 1.0);
+    const double step = D == 64 ? (w == 4 ? 1.55 : 1.65) : (w == 4 ? 2.2 : 3.0);
+    double t;
+    if (D == 64 && w == 4)   // two workgroups share a CU
+      t = start + std::max(1.0, items) * (steps * step + 0.6);
+    else
+      t = std::ceil(items) * (start + (D == 128 && w == 2 ? 0.8 : 0.2) + steps * step);
+    if (t < best) {
+      best = t;
+      qw = w;
+    }
+  }
+  return qw;
 }
 
 template <AttnType T, int D>
@@ -568,7 +810,17 @@ hipError_t run(const AttnDesc& d, hipStream_t s) {
   if (span >= (1ll << 31)) return hipErrorNotSupported;
   // item indices are 32-bit in the kernel
   if ((int64_t)d.B * d.H * p.qtiles > 0x7fffffff) return hipErrorInvalidValue;
+  // (a cycle probe's slots are counted for attn_fwd)
+  const int qw = d.probe ? 0 : split_blocks((int64_t)d.B * d.H, d.S, D, p.causal);
+  if (qw) {
+    p.qtiles = (d.S + 32 * qw - 1) / (32 * qw);
+    const dim3 grid((unsigned)(p.heads * p.qtiles));
+    if (qw == 4) hipLaunchKernelGGL((attn_split<T, D, 4, 2>), grid, dim3(64 * kNW), 0, s, p);
+    else hipLaunchKernelGGL((attn_split<T, D, 2, D == 64 ? 2 : 1>), grid, dim3(64 * kNW), 0, s, p);
+    return hipGetLastError();
+  }
   const int64_t wgs = workgroups(d.B, d.H, d.S);
+  p.hb = heads_per_block((p.heads + 7) / 8, p.qtiles, (int)(wgs / 8), p.causal);
   hipLaunchKernelGGL((attn_fwd<T, D>), dim3((unsigned)wgs), dim3(64 * kNW), 0, s, p);
   return hipGetLastError();
 }

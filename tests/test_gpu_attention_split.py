@@ -1,0 +1,63 @@
+"""Attention problems of few query tiles: items of 128 or 64 queries whose
+workgroups split the keys over two or four groups of waves (attn_split), and
+causal launches whose heads form one block of the persistent kernel's item
+order. Every head against the oracle."""
+import numpy as np
+import pytest
+
+import grxcp_amd as g
+import oracle as O
+from helpers import normwise_rel_err
+from test_gpu_dnn import run_attention
+
+pytestmark = pytest.mark.gpu
+BF16, F16 = g.GRX_R_16BF, g.GRX_R_16F
+
+
+def check_heads(dnn, t, B, H, S, D, causal):
+    o, q, k, v = run_attention(dnn, t, B, H, S, D, causal, seed=S + D + H)
+    assert np.isfinite(o).all()
+    for b in range(B):
+        for h in range(H):
+            ref = O.attention_head(q[b, h], k[b, h], v[b, h], causal, D ** -0.5)
+            assert normwise_rel_err(o[b, h], ref) <= 1e-2, (b, h)
+
+
+# S around the tiles (64 keys), the steps (128 and 256 keys) and the items (64
+# and 128 queries): key groups without a tile, partial tiles, one and several
+# steps; few heads (64-query items) and more (128-query items)
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,S", [(1, 1, 1), (1, 3, 63), (2, 4, 65), (1, 8, 129), (1, 5, 257), (1, 4, 700),
+                                   (1, 24, 200), (2, 16, 300), (3, 20, 130), (1, 32, 517), (1, 8, 1025)])
+def test_attention_split(dnn, B, H, S, D, causal):
+    check_heads(dnn, BF16, B, H, S, D, causal)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_attention_split_f16(dnn, D):
+    check_heads(dnn, F16, 1, 12, 321, D, True)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("case", ["growing", "shrinking"])
+def test_attention_split_groups_with_unlike_maxima(dnn, case, D):
+    """Key magnitudes that grow or shrink along the sequence: the groups'
+    maxima differ by far more than a float's exponent range in their weights,
+    so all but one group's contribution underflows."""
+    B, H, S = 1, 4, 640
+    r = np.random.default_rng(11 + D)
+    ramp = np.linspace(0.0, 40.0, S, dtype=np.float32)[None, None, :, None]
+    k = r.standard_normal((B, H, S, D)).astype(np.float32) * (ramp if case == "growing" else ramp[:, :, ::-1])
+    o, q, kq, v = run_attention(dnn, BF16, B, H, S, D, False, seed=5, k=k)
+    assert np.isfinite(o).all()
+    for h in range(H):
+        ref = O.attention_head(q[0, h], kq[0, h], v[0, h], False, D ** -0.5)
+        assert normwise_rel_err(o[0, h], ref) <= 1e-2, h
+
+
+@pytest.mark.parametrize("H,S,D", [(104, 760, 64), (88, 700, 128)])
+def test_attention_heads_in_one_block(dnn, H, S, D):
+    """39 and 33 causal items on each XCD's 32 workgroups: one block of all
+    its heads, dealt in a snake from the heaviest items on."""
+    check_heads(dnn, BF16, 1, H, S, D, True)
