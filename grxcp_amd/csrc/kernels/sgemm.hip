@@ -20,10 +20,18 @@
 #include "../launch.h"
 #include "device_common.h"
 
+#include <algorithm>
+#include <type_traits>
+
 namespace grxk {
 namespace {
 
 constexpr int kK = 16;   // K per stage
+
+// Four consecutive floats at any 4-byte aligned address: one
+// global_load_dwordx4, which gfx950 takes on dword alignment, so columns of an
+// odd leading dimension are read 16 bytes at a time too.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 struct SParams {
   const float* a; const float* b; float* c;
@@ -45,11 +53,11 @@ struct SParams {
 // barrier per stage. An MFMA k-step reads one float per lane per operand:
 // lane l takes row/column l%32 at k = 2s + l/32.
 // TA/TB are template parameters, so the staging code has no run-time
-// transpose switch. VEC: leading dimensions, strides and base pointers are
-// multiples of 4 floats, so 4 consecutive elements along an operand's
-// contiguous dimension are one aligned 16-byte load; a stage wholly inside
-// the matrices (decided once per stage, uniformly) takes those loads with no
-// per-element guard, other stages the guarded path. (Measured at 4096^3:
+// transpose switch. 4 consecutive elements along an operand's contiguous
+// dimension are one 16-byte load at float alignment, whatever the leading
+// dimension; a stage wholly inside the matrices (decided once per stage,
+// uniformly) takes those loads with no per-element guard, other stages the
+// guarded path. (Measured at 4096^3:
 // 91 -> 129 TFLOP/s against one kernel with run-time transposes and guards,
 // 129 -> 134 with the fragment reads one k-step ahead. Slower, same output:
 // a pitch that puts k-rows 2s and 2s+1 half the banks apart (3 %: 3 instead
@@ -64,10 +72,10 @@ struct SParams {
 // conflicted -- the fragment reads (four 16-lane groups at k = 4s .. 4s+3),
 // the transposing stores of a K-contiguous operand (8-way at a pitch of 48)
 // and the direct stores (4-way at 48); 512^3 30.7 -> 32.0 TFLOP/s.
-template <int MT, bool VEC, bool TA, bool TB>
+template <int MT, int KK, bool TA, bool TB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void sgemm_mfma(SParams p) {
-  constexpr int kK = MT == 32 ? 32 : grxk::kK;   // K per stage
+  constexpr int kK = KK;                // K per stage
   constexpr int WT = MT / 2;            // wave tile edge
   constexpr int NF = WT / 32;           // 32x32 MFMA tiles per wave edge (0 at MT = 32)
   constexpr int PITCH = MT == 32 ? 33 : MT + 4;  // MT + 4: 16-byte aligned rows, 4 workgroups fit a CU's LDS at MT=128
@@ -96,33 +104,62 @@ void sgemm_mfma(SParams p) {
   constexpr int GPT = PER / 4;  // groups per thread per operand
   float ra[PER], rb[PER];
   // Element (c, o) of a group is X[o*ld + c], valid iff c < lim_cont, o < lim_other.
-  auto load_group = [&](const float* X, int64_t ld, bool full, int lim_cont, int lim_other,
+  auto load_group = [&](const float* X, int64_t ld, int lim_cont, int lim_other,
                         int cont, int other, float* out) {
     const float* q = X + (int64_t)other * ld + cont;
-    if (VEC && (full || (other < lim_other && cont + 3 < lim_cont))) {
-      const float4 v = *(const float4*)q;
-      out[0] = v.x; out[1] = v.y; out[2] = v.z; out[3] = v.w;
+    if (other < lim_other && cont + 3 < lim_cont) {
+      const f32x4 v = *(const f32x4u*)q;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) out[e] = v[e];
     } else {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) out[v] = (other < lim_other && cont + v < lim_cont) ? q[v] : 0.0f;
+      for (int e = 0; e < 4; ++e) out[e] = (other < lim_other && cont + e < lim_cont) ? q[e] : 0.0f;
     }
   };
   // op(A) (m x k): N stores A[k*lda + i] (cont = i), T stores A[i*lda + k] (cont = k).
   // op(B) (k x n): N stores B[j*ldb + k] (cont = k), T stores B[k*ldb + j] (cont = j).
-  auto load_all = [&](int k0, bool full) __attribute__((always_inline)) {
+  // Where each group starts in the first stage, for stages read without
+  // guards. Groups wholly past m (n) read the tile's first row (column)
+  // instead: what they hold only reaches rows and columns of C that are not
+  // stored.
+  const float* ga[GPT];
+  const float* gb[GPT];
 #pragma unroll
-    for (int q = 0; q < GPT; ++q) {
-      const int e = 4 * (tid + 256 * q);
-      if (TA) load_group(A, p.lda, full, p.k, p.m, k0 + e % kK, row0 + e / kK, &ra[4 * q]);
-      else load_group(A, p.lda, full, p.m, p.k, row0 + e % MT, k0 + e / MT, &ra[4 * q]);
-      if (TB) load_group(B, p.ldb, full, p.n, p.k, col0 + e % MT, k0 + e / MT, &rb[4 * q]);
-      else load_group(B, p.ldb, full, p.k, p.n, k0 + e % kK, col0 + e / kK, &rb[4 * q]);
-    }
-  };
+  for (int q = 0; q < GPT; ++q) {
+    const int e = 4 * (tid + 256 * q);
+    const int ia = TA ? e / kK : e % MT, ka = TA ? e % kK : e / MT;
+    const int ib = TB ? e % MT : e / kK, kb = TB ? e / MT : e % kK;
+    const int64_t i = row0 + ia < p.m ? row0 + ia : row0, j = col0 + ib < p.n ? col0 + ib : col0;
+    ga[q] = A + (TA ? i * p.lda + ka : ka * p.lda + i);
+    gb[q] = B + (TB ? kb * p.ldb + j : j * p.ldb + kb);
+  }
+  // A group that straddles m (n) along memory reads up to 3 floats past it:
+  // the next columns' (rows') values, inside the operand while at least 3
+  // floats of later k follow.
+  const int64_t slack_ld = !TA && TB ? min(p.lda, p.ldb) : TB ? p.ldb : p.lda;
   auto load = [&](int k0) {
     // One uniform decision per stage: the unguarded path is straight-line code.
-    if (VEC && interior && k0 + kK <= p.k) load_all(k0, true);
-    else load_all(k0, false);
+    if (k0 + kK <= p.k && (interior || (TA && !TB) || (p.k - k0 - kK) * slack_ld >= 3)) {
+#pragma unroll
+      for (int q = 0; q < GPT; ++q) {
+        const f32x4 va = *(const f32x4u*)(ga[q] + (TA ? (int64_t)k0 : k0 * p.lda));
+        const f32x4 vb = *(const f32x4u*)(gb[q] + (TB ? k0 * p.ldb : (int64_t)k0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          ra[4 * q + e] = va[e];
+          rb[4 * q + e] = vb[e];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < GPT; ++q) {
+        const int e = 4 * (tid + 256 * q);
+        if (TA) load_group(A, p.lda, p.k, p.m, k0 + e % kK, row0 + e / kK, &ra[4 * q]);
+        else load_group(A, p.lda, p.m, p.k, row0 + e % MT, k0 + e / MT, &ra[4 * q]);
+        if (TB) load_group(B, p.ldb, p.n, p.k, col0 + e % MT, k0 + e / MT, &rb[4 * q]);
+        else load_group(B, p.ldb, p.k, p.n, k0 + e % kK, col0 + e / kK, &rb[4 * q]);
+      }
+    }
   };
   auto store = [&](int buf) {
 #pragma unroll
@@ -295,11 +332,6 @@ __global__ void sscal_kernel(int n, float alpha, float* x, int incx, grxCycleSlo
   l12_record(probe, t0);
 }
 
-// Four consecutive floats at any 4-byte aligned address: one
-// global_load_dwordx4, which gfx950 takes on dword alignment, so columns of an
-// odd leading dimension are read 16 bytes at a time too.
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-
 // Element i of a BLAS vector of n elements lies at base + i * inc.
 __device__ __forceinline__ int64_t blas_base(int n, int inc) {
   return inc > 0 ? 0 : (int64_t)(n - 1) * (-(int64_t)inc);
@@ -470,38 +502,19 @@ hipError_t launch_sgemm(const SgemmDesc& d, hipStream_t s) {
   p.tiles_m = (d.m + mt - 1) / mt;
   const int64_t tiles = (int64_t)p.tiles_m * ((d.n + mt - 1) / mt);
   if (tiles > 0x7fffffff) return hipErrorInvalidValue;
-  const bool vec = d.lda % 4 == 0 && d.ldb % 4 == 0 && d.stride_a % 4 == 0 && d.stride_b % 4 == 0 &&
-                   (uintptr_t)d.a % 16 == 0 && (uintptr_t)d.b % 16 == 0;
   const dim3 grid((unsigned)tiles, 1, (unsigned)d.batch);
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, p); };
-  const int sel = (mt == 128 ? 8 : mt == 32 ? 16 : 0) | (vec ? 4 : 0) | (d.ta ? 2 : 0) | (d.tb ? 1 : 0);
-  switch (sel) {
-    case 16: go(sgemm_mfma<32, false, false, false>); break;
-    case 17: go(sgemm_mfma<32, false, false, true>); break;
-    case 18: go(sgemm_mfma<32, false, true, false>); break;
-    case 19: go(sgemm_mfma<32, false, true, true>); break;
-    case 20: go(sgemm_mfma<32, true, false, false>); break;
-    case 21: go(sgemm_mfma<32, true, false, true>); break;
-    case 22: go(sgemm_mfma<32, true, true, false>); break;
-    case 23: go(sgemm_mfma<32, true, true, true>); break;
-    case 0:  go(sgemm_mfma<64, false, false, false>); break;
-    case 1:  go(sgemm_mfma<64, false, false, true>); break;
-    case 2:  go(sgemm_mfma<64, false, true, false>); break;
-    case 3:  go(sgemm_mfma<64, false, true, true>); break;
-    case 4:  go(sgemm_mfma<64, true, false, false>); break;
-    case 5:  go(sgemm_mfma<64, true, false, true>); break;
-    case 6:  go(sgemm_mfma<64, true, true, false>); break;
-    case 7:  go(sgemm_mfma<64, true, true, true>); break;
-    case 8:  go(sgemm_mfma<128, false, false, false>); break;
-    case 9:  go(sgemm_mfma<128, false, false, true>); break;
-    case 10: go(sgemm_mfma<128, false, true, false>); break;
-    case 11: go(sgemm_mfma<128, false, true, true>); break;
-    case 12: go(sgemm_mfma<128, true, false, false>); break;
-    case 13: go(sgemm_mfma<128, true, false, true>); break;
-    case 14: go(sgemm_mfma<128, true, true, false>); break;
-    case 15: go(sgemm_mfma<128, true, true, true>); break;
-    default: return hipErrorInvalidValue;
-  }
+  auto go_mt = [&](auto mt_c) {
+    constexpr int MT = decltype(mt_c)::value;
+    constexpr int KK = MT == 32 ? 32 : 16;   // K per stage
+    if (d.ta && d.tb) go(sgemm_mfma<MT, KK, true, true>);
+    else if (d.ta) go(sgemm_mfma<MT, KK, true, false>);
+    else if (d.tb) go(sgemm_mfma<MT, KK, false, true>);
+    else go(sgemm_mfma<MT, KK, false, false>);
+  };
+  if (mt == 128) go_mt(std::integral_constant<int, 128>{});
+  else if (mt == 64) go_mt(std::integral_constant<int, 64>{});
+  else go_mt(std::integral_constant<int, 32>{});
   return hipGetLastError();
 }
 
