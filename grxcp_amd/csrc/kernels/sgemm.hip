@@ -4,10 +4,10 @@
 // Sgemm replaces the reference's one-thread-per-output kernel
 // (ref: src/libs/grxblas/kernels/sgemm.cpp:22-89; 2 global loads per
 // multiply-add) with an fp32 matrix-core kernel (v_mfma_f32_32x32x2_f32): a
-// 128x128 (or, for problems too small to fill the chip, 64x64) tile of C per
-// 256-thread workgroup, 16-deep K stages double-buffered through LDS with
-// guarded loads that apply op() while staging (all four transposes, ragged
-// shapes, any leading dimension). The batch is the grid's z dimension with
+// 128x128 (or, for problems too small to fill the chip, 64x64 or 32x32) tile
+// of C per workgroup, 16- or 32-deep K stages double-buffered through LDS with
+// loads that apply op() while staging (all four transposes, ragged shapes,
+// any leading dimension). The batch is the grid's z dimension with
 // signed element strides (a zero stride broadcasts an operand), exactly the
 // reference's one-launch batching (ref: src/libs/grxblas/grxblas.cpp:936-938).
 // beta == 0 never reads C (ref: kernels/sgemm.cpp:80-85). Problems that
@@ -26,8 +26,6 @@
 namespace grxk {
 namespace {
 
-constexpr int kK = 16;   // K per stage
-
 // Four consecutive floats at any 4-byte aligned address: one
 // global_load_dwordx4, which gfx950 takes on dword alignment, so columns of an
 // odd leading dimension are read 16 bytes at a time too.
@@ -44,9 +42,9 @@ struct SParams {
   grxCycleSlot* probe;
 };
 
-// One workgroup = 4 waves (2 x 2) computes an MT x MT tile of C with
+// 4 waves (2 x 2) compute an MT x MT tile of C with
 // v_mfma_f32_32x32x2_f32 (each wave MT/2 x MT/2, i.e. (MT/64)^2 .. 4 MFMA
-// tiles). K advances 16 at a time through double-buffered LDS tiles
+// tiles). K advances KK at a time through double-buffered LDS tiles
 // As[kk][i] = op(A)[row0+i][k0+kk] and Bs[kk][j] = op(B)[k0+kk][col0+j]; the
 // next stage's loads (op() applied while loading, zeros outside the matrix)
 // are issued before the current stage's MFMAs and stored after them, one
@@ -65,26 +63,47 @@ struct SParams {
 // stages (2 workgroups per CU, 5-9 %), 256x256 tiles (one wave per SIMD,
 // 4 %), the next stage's LDS stores moved to mid-stage (no change).)
 //
+// KG K groups of 4 waves share a tile: group g takes stages g, g + KG, ...
+// in LDS buffers of its own, and their accumulators meet pairwise in LDS at
+// the end, in group 0, which stores C. It puts more waves on a CU where there
+// are few tiles, whose stages would otherwise wait for one load each (1024^3,
+// one 64x64 tile per CU: 29.8 us with KG = 1, 27 with 2, 25.7 with 4; two
+// stages of loads in flight per group instead: no change).
+//
+// Tiles at the edge of C read their stages without guards too: rows past m
+// (columns past n) of a group repeat the tile's first, and what a group reads
+// past m or n along memory stays in its own rows of the product, none of which
+// are stored. Guards remain where a stage passes k or the operand's end
+// (1000^3 51.8 -> 29.8 us, 4095^3 1616 -> 1099; before, the waves of an edge
+// tile took the guarded element loads, and waited for them, in every stage).
+//
 // MT = 32 (problems of few 64x64 tiles, 512^3 among them): each wave one
 // 16x16 tile with v_mfma_f32_16x16x4_f32, K 32 deep per stage (so that the
 // staging keeps one 4-element group per thread and operand), rows 33 floats
 // apart: over 64 banks that keeps every access of the tile at most 2-way
 // conflicted -- the fragment reads (four 16-lane groups at k = 4s .. 4s+3),
 // the transposing stores of a K-contiguous operand (8-way at a pitch of 48)
-// and the direct stores (4-way at 48); 512^3 30.7 -> 32.0 TFLOP/s.
-template <int MT, int KK, bool TA, bool TB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
+// and the direct stores (4-way at 48); 512^3 30.7 -> 32.0 TFLOP/s, 39 with
+// the K groups.
+template <int MT, int KK, int KG, bool TA, bool TB>
+__global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void sgemm_mfma(SParams p) {
   constexpr int kK = KK;                // K per stage
   constexpr int WT = MT / 2;            // wave tile edge
   constexpr int NF = WT / 32;           // 32x32 MFMA tiles per wave edge (0 at MT = 32)
   constexpr int PITCH = MT == 32 ? 33 : MT + 4;  // MT + 4: 16-byte aligned rows, 4 workgroups fit a CU's LDS at MT=128
   constexpr int PER = MT * kK / 256;    // elements per thread per operand per stage
-  __shared__ float As[2][kK][PITCH];
-  __shared__ float Bs[2][kK][PITCH];
+  constexpr int kAcc = MT * MT / 256;   // accumulators per thread
+  constexpr int kStages = KG * 2 * kK * PITCH;
+  constexpr int kMerge = KG > 1 ? KG / 2 * MT * MT : 0;
+  // [operand][K group][stage parity][k][row], later the groups' partial sums
+  __shared__ float smem[2 * kStages > kMerge ? 2 * kStages : kMerge];
+  const int kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  float (*As)[kK][PITCH] = (float (*)[kK][PITCH])smem + 2 * kg;
+  float (*Bs)[kK][PITCH] = (float (*)[kK][PITCH])smem + 2 * KG + 2 * kg;
 
   const uint64_t t0 = p.probe ? cycle_now() : 0;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x & 255;    // within the K group
   const int lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
   const int wm = wave & 1, wn = wave >> 1;
@@ -175,6 +194,30 @@ void sgemm_mfma(SParams p) {
     }
   };
 
+  auto first = [&]() __attribute__((always_inline)) {
+    if (kg * kK < p.k || kg == 0) {
+      load(kg * kK);
+      store(0);
+    }
+    __syncthreads();
+  };
+  // Sum of the K groups' accumulators, at(0 .. kAcc-1) of each thread, in
+  // group 0, pairwise; false in the groups that are done.
+  auto merge = [&](auto at) __attribute__((always_inline)) {
+#pragma unroll
+    for (int half = KG / 2; half >= 1; half /= 2) {
+      if (kg >= half && kg < 2 * half)
+#pragma unroll
+        for (int e = 0; e < kAcc; ++e) smem[((kg - half) * kAcc + e) * 256 + tid] = at(e);
+      __syncthreads();
+      if (kg < half)
+#pragma unroll
+        for (int e = 0; e < kAcc; ++e) at(e) += smem[(kg * kAcc + e) * 256 + tid];
+      if (half > 1) __syncthreads();
+    }
+    return kg == 0;
+  };
+
   // C = alpha*acc + beta*C (col-major) for a lane's run of 4 rows i0.. of
   // column gj: one 16-byte non-temporal store where the run lies inside C and
   // C's columns are 16-byte aligned, element by element otherwise (same
@@ -208,26 +251,27 @@ void sgemm_mfma(SParams p) {
     // column l%16 of the result.
     const int r16 = lane & 15, kq = lane >> 4;
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    load(0);
-    store(0);
-    __syncthreads();
     int buf = 0;
-    for (int k0 = 0; k0 < p.k; k0 += kK) {
-      const bool more = k0 + kK < p.k;
-      if (more) load(k0 + kK);
+    first();
+    for (int kb = 0; kb < p.k; kb += KG * kK) {
+      const int k0 = kb + kg * kK;
+      const bool more = k0 + KG * kK < p.k;
+      if (more) load(k0 + KG * kK);
       float av[kK / 4], bv[kK / 4];
 #pragma unroll
       for (int st = 0; st < kK / 4; ++st) {
         av[st] = As[buf][4 * st + kq][16 * wm + r16];
         bv[st] = Bs[buf][4 * st + kq][16 * wn + r16];
       }
+      if (k0 < p.k)
 #pragma unroll
-      for (int st = 0; st < kK / 4; ++st)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[st], bv[st], acc, 0, 0, 0);
+        for (int st = 0; st < kK / 4; ++st)
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[st], bv[st], acc, 0, 0, 0);
       if (more) store(buf ^ 1);
       __syncthreads();
       buf ^= 1;
     }
+    if (!merge([&](int e) -> float& { return ((float*)&acc)[e]; })) return;
     const int gj = col0 + 16 * wn + r16;
     const int i0 = row0 + 16 * wm + 4 * kq;
     if (gj < p.n && i0 < p.m) {
@@ -243,44 +287,46 @@ void sgemm_mfma(SParams p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[fm][fn][r] = 0.0f;
 
-    load(0);
-    store(0);
-    __syncthreads();
     int buf = 0;
-    for (int k0 = 0; k0 < p.k; k0 += kK) {
-      const bool more = k0 + kK < p.k;
-      if (more) load(k0 + kK);
+    first();
+    for (int kb = 0; kb < p.k; kb += KG * kK) {
+      const int k0 = kb + kg * kK;
+      const bool more = k0 + KG * kK < p.k;
+      if (more) load(k0 + KG * kK);
       // Fragments one k-step ahead: step s+1's LDS reads are issued before
       // step s's MFMAs (the scheduling barriers keep that order), so each
       // wait covers reads issued a whole step earlier.
       float av[2][NF], bv[2][NF];
+      if (k0 < p.k) {
 #pragma unroll
-      for (int f = 0; f < NF; ++f) {
-        av[0][f] = As[buf][hh][WT * wm + 32 * f + l32];
-        bv[0][f] = Bs[buf][hh][WT * wn + 32 * f + l32];
-      }
-#pragma unroll
-      for (int s = 0; s < kK / 2; ++s) {
-        if (s + 1 < kK / 2) {
-#pragma unroll
-          for (int f = 0; f < NF; ++f) {
-            av[(s + 1) & 1][f] = As[buf][2 * s + 2 + hh][WT * wm + 32 * f + l32];
-            bv[(s + 1) & 1][f] = Bs[buf][2 * s + 2 + hh][WT * wn + 32 * f + l32];
-          }
+        for (int f = 0; f < NF; ++f) {
+          av[0][f] = As[buf][hh][WT * wm + 32 * f + l32];
+          bv[0][f] = Bs[buf][hh][WT * wn + 32 * f + l32];
         }
-        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int fm = 0; fm < NF; ++fm)
+        for (int s = 0; s < kK / 2; ++s) {
+          if (s + 1 < kK / 2) {
 #pragma unroll
-          for (int fn = 0; fn < NF; ++fn)
-            acc[fm][fn] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[s & 1][fm], bv[s & 1][fn], acc[fm][fn],
-                                                               0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
+            for (int f = 0; f < NF; ++f) {
+              av[(s + 1) & 1][f] = As[buf][2 * s + 2 + hh][WT * wm + 32 * f + l32];
+              bv[(s + 1) & 1][f] = Bs[buf][2 * s + 2 + hh][WT * wn + 32 * f + l32];
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int fm = 0; fm < NF; ++fm)
+#pragma unroll
+            for (int fn = 0; fn < NF; ++fn)
+              acc[fm][fn] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[s & 1][fm], bv[s & 1][fn], acc[fm][fn],
+                                                                 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
       if (more) store(buf ^ 1);
       __syncthreads();
       buf ^= 1;
     }
+    if (!merge([&](int e) -> float& { return ((float*)acc)[e]; })) return;
 
     // A lane holds column l32 of each MFMA tile and rows 8*(r/4) + 4*hh +
     // r%4: runs of 4 rows.
@@ -493,29 +539,41 @@ hipError_t launch_sgemm(const SgemmDesc& d, hipStream_t s) {
   p.alpha = d.alpha; p.beta = d.beta;
   p.probe = d.probe;
   if (d.batch > 65535) return hipErrorInvalidValue;
-  // 128-wide tiles once they fill the chip, 64-wide below that, 32-wide
-  // where 64-wide tiles would leave half the CUs idle (without a cycle
-  // probe, whose slots are counted for 64x64 tiles).
+  // Tile and K groups. 128-wide tiles (four workgroups share a CU) where they
+  // are three or more per CU: 4095^3 1099 us, 1143 with 64-wide ones; below
+  // that 64-wide tiles waste less of the last round (2047^2 x 500, 256 or 1024
+  // tiles: 56 / 47 us), and where those are fewer than the CUs, 32-wide ones
+  // (512^3 6.8 / 14.0 us, 700^3 13.4 / 18.9). Two K groups overlap one's loads
+  // with the other's products; four where a CU has at most about one tile
+  // (1000^3 28 -> 26 us, 256^2 x 2048 18.5 -> 16.4; 30.0 with one). A cycle
+  // probe's slots are counted for 64-wide tiles and one group.
   const int64_t big = ((int64_t)(d.m + 127) / 128) * ((d.n + 127) / 128) * d.batch;
   const int64_t mid = ((int64_t)(d.m + 63) / 64) * ((d.n + 63) / 64) * d.batch;
-  const int mt = big >= 256 ? 128 : (mid >= 128 || d.probe ? 64 : 32);
-  p.tiles_m = (d.m + mt - 1) / mt;
-  const int64_t tiles = (int64_t)p.tiles_m * ((d.n + mt - 1) / mt);
-  if (tiles > 0x7fffffff) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)tiles, 1, (unsigned)d.batch);
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, p); };
-  auto go_mt = [&](auto mt_c) {
-    constexpr int MT = decltype(mt_c)::value;
-    constexpr int KK = MT == 32 ? 32 : 16;   // K per stage
-    if (d.ta && d.tb) go(sgemm_mfma<MT, KK, true, true>);
-    else if (d.ta) go(sgemm_mfma<MT, KK, true, false>);
-    else if (d.tb) go(sgemm_mfma<MT, KK, false, true>);
-    else go(sgemm_mfma<MT, KK, false, false>);
+  const int64_t small = ((int64_t)(d.m + 31) / 32) * ((d.n + 31) / 32) * d.batch;
+  auto go = [&](auto mt_c, auto kg_c) {
+    constexpr int MT = decltype(mt_c)::value, KG = decltype(kg_c)::value, KK = MT == 32 ? 32 : 16;
+    p.tiles_m = (d.m + MT - 1) / MT;
+    const int64_t tiles = (int64_t)p.tiles_m * ((d.n + MT - 1) / MT);
+    if (tiles > 0x7fffffff) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)tiles, 1, (unsigned)d.batch);
+    auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256 * KG), 0, s, p); };
+    if (d.ta && d.tb) launch(sgemm_mfma<MT, KK, KG, true, true>);
+    else if (d.ta) launch(sgemm_mfma<MT, KK, KG, true, false>);
+    else if (d.tb) launch(sgemm_mfma<MT, KK, KG, false, true>);
+    else launch(sgemm_mfma<MT, KK, KG, false, false>);
+    return hipGetLastError();
   };
-  if (mt == 128) go_mt(std::integral_constant<int, 128>{});
-  else if (mt == 64) go_mt(std::integral_constant<int, 64>{});
-  else go_mt(std::integral_constant<int, 32>{});
-  return hipGetLastError();
+  using std::integral_constant;
+  constexpr integral_constant<int, 128> t128;
+  constexpr integral_constant<int, 64> t64;
+  constexpr integral_constant<int, 32> t32;
+  constexpr integral_constant<int, 1> g1;
+  constexpr integral_constant<int, 2> g2;
+  constexpr integral_constant<int, 4> g4;
+  if (d.probe) return big >= 256 ? go(t128, g1) : go(t64, g1);
+  if (big >= 768) return go(t128, g1);
+  if (mid >= 256) return mid <= 384 && d.k > 128 ? go(t64, g4) : go(t64, g2);
+  return small <= 512 && d.k > 128 ? go(t32, g4) : go(t32, g2);
 }
 
 int64_t l1_blocks(int n) { return std::min<int64_t>(((int64_t)n + 255) / 256, 65536); }

@@ -57,6 +57,19 @@ def test_sgemm_larger_ragged_all_transposes(blas):
             assert run_case(blas, ta, tb, 133, 97, 150, 1.0, 0.5, 5) == (0, 0)
 
 
+# Tiles of 32, 64 and 128 with one, two and four K groups; m and n below, at and
+# past a tile's edge (and below 4: a 16-byte read past m spans columns), K
+# below, at and past a stage, and K groups left without one.
+@pytest.mark.parametrize("ta", [0, 1])
+@pytest.mark.parametrize("tb", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (2, 3, 64), (3, 2, 131), (33, 31, 129), (64, 32, 256), (511, 513, 96),
+                                   (700, 690, 130), (1030, 1001, 160), (1100, 1500, 48), (3585, 3586, 20)])
+def test_sgemm_tiles_and_k_groups(blas, ta, tb, m, n, k):
+    assert run_case(blas, ta, tb, m, n, k, 1.0, 0.0, 0) == (0, 0)
+    if m * n < 1 << 20:
+        assert run_case(blas, ta, tb, m, n, k, -1.5, 0.5, 3) == (0, 0)
+
+
 def run_batched(blas, ta, tb, m, n, k, alpha, beta, batch, gap, broadcast_b):
     """ref test_grxblas.cpp:88-172"""
     lda, ldb, ldc = max(1, k if ta else m), max(1, n if tb else k), max(1, m)
