@@ -64,6 +64,10 @@ struct OpBF16 {
   __device__ static void mma16(i32x4 a, i32x4 b, Acc16& c) {
     asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
   }
+  __device__ static Acc16 mul16(i32x4 a, i32x4 b, Acc16 c) {   // scheduled by the compiler
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
 };
 
 struct OpF16 {
@@ -83,6 +87,10 @@ struct OpF16 {
   __device__ static void mma16(i32x4 a, i32x4 b, Acc16& c) {
     asm("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
   }
+  __device__ static Acc16 mul16(i32x4 a, i32x4 b, Acc16 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
 };
 
 struct OpI8 {
@@ -100,6 +108,9 @@ struct OpI8 {
   using Acc16 = i32x4;
   __device__ static void mma16(i32x4 a, i32x4 b, Acc16& c) {
     asm("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  }
+  __device__ static Acc16 mul16(i32x4 a, i32x4 b, Acc16 c) {
+    return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
   }
 };
 
@@ -296,6 +307,36 @@ __device__ __forceinline__ void store_run(const KParams& p, int i0, int j, const
   }
 }
 
+// Rows i0 .. i0+3 of column j (i0 < m, j < n, i0 a multiple of 4), each value
+// as Epi<OUT>::put_run rounds it. `vec`: C's columns are 16-byte aligned, so
+// four rows are one 8- or 16-byte store.
+template <MmaOut OUT, bool STREAM, class E>
+__device__ __forceinline__ void store4(const KParams& p, int i0, int j, const E* v, bool vec) {
+  using P = Epi<OUT>;
+  using T = typename P::T;
+  if constexpr (P::kRun == 4) {
+    store_run<OUT, STREAM>(p, i0, j, v, 4, vec);
+  } else if (vec && i0 + 4 <= p.m) {
+    T* c = (T*)p.c + (int64_t)j * p.ldc + i0;
+    u32x2 o;
+    if constexpr (OUT == MmaOut::DEQ_BF16) {
+      const float s = p.scale[j];
+      o[0] = pack_bf16x2(__fmul_rn((float)v[0], s), __fmul_rn((float)v[1], s));
+      o[1] = pack_bf16x2(__fmul_rn((float)v[2], s), __fmul_rn((float)v[3], s));
+    } else if (p.beta == 0.0f) {
+      o[0] = P::pack(__fmul_rn(p.alpha, v[0]), __fmul_rn(p.alpha, v[1]));
+      o[1] = P::pack(__fmul_rn(p.alpha, v[2]), __fmul_rn(p.alpha, v[3]));
+    } else {
+      const u32x2 old = *(const u32x2*)c;
+      o[0] = P::pack(P::apply(p, v[0], (uint16_t)(old[0] & 0xffff)), P::apply(p, v[1], (uint16_t)(old[0] >> 16)));
+      o[1] = P::pack(P::apply(p, v[2], (uint16_t)(old[1] & 0xffff)), P::apply(p, v[3], (uint16_t)(old[1] >> 16)));
+    }
+    *(u32x2*)c = o;
+  } else {
+    store_run<OUT, STREAM>(p, i0, j, v, 4, false);
+  }
+}
+
 // Spread a 32x32 accumulator tile (rows base_i.., cols base_j..) to C, four
 // rows per lane and store (general path: no alignment assumed).
 template <class Op, MmaOut OUT>
@@ -385,6 +426,17 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef int i32x2 __attribute__((ext_vector_type(2)));
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
+
+// The four words of a raw buffer descriptor, for assembly.
+__device__ __forceinline__ i32x4 rsrc_words(const uint8_t* base, int bytes) {
+  const uint64_t a = (uint64_t)(uintptr_t)base;
+  i32x4 r;
+  r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)a);
+  r[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32) & 0xffff);
+  r[2] = __builtin_amdgcn_readfirstlane(bytes);
+  r[3] = (int)kRsrcWord3;
+  return r;
+}
 
 template <class Op, MmaOut OUT, bool STREAM = true>
 __global__ __launch_bounds__(256, 1) void gemm_tn_fast(KParams batch_p) {
@@ -975,15 +1027,6 @@ __global__ __launch_bounds__(256, NS == 2 ? 2 : 1) void gemm_tn128(KParams batch
   constexpr int kRowsAN = kFastKBytes / EB;               // k-rows of an AN stage (64 or 128)
   constexpr int kRowChunks = kT128 * EB / 16;             // 16-byte chunks of a k-row (16 or 8)
   constexpr int kRowsDma = 64 / kRowChunks;               // k-rows per 1 KB DMA block (4 or 8)
-  auto rsrc_words = [&](const uint8_t* base, int bytes) {
-    const uint64_t a = (uint64_t)(uintptr_t)base;
-    i32x4 r;
-    r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)a);
-    r[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32) & 0xffff);
-    r[2] = __builtin_amdgcn_readfirstlane(bytes);
-    r[3] = (int)kRsrcWord3;
-    return r;
-  };
   // AN: from the tile's first m; every k-row of A, to the end of the matrix
   // (m past the matrix within a row reads the next row's values, which only
   // reach rows of C that are never stored). BN likewise from the first n.
@@ -1167,7 +1210,6 @@ __global__ __launch_bounds__(256, NS == 2 ? 2 : 1) void gemm_tn128(KParams batch
 
   // Lane l holds rows 16i + 4*(l/16) .. +3 of column 16j + l%16.
   using E = typename Op::Elem;
-  using T = typename Epi<OUT>::T;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -1176,33 +1218,142 @@ __global__ __launch_bounds__(256, NS == 2 ? 2 : 1) void gemm_tn128(KParams batch
       const int i0 = row0 + wm * 64 + 16 * i + 4 * (lane >> 4);
       if (gj >= p.n || i0 >= p.m) continue;
       const E v[4] = {(E)acc[i][j][0], (E)acc[i][j][1], (E)acc[i][j][2], (E)acc[i][j][3]};
-      if constexpr (Epi<OUT>::kRun == 4) {
-        store_run<OUT, STREAM>(p, i0, gj, v, 4, true);
-      } else if (i0 + 4 <= p.m) {
-        // 16-bit C: the run's 8 bytes, each value as Epi<OUT>::put_run
-        // (or put_run_scaled) rounds it.
-        T* c = (T*)p.c + (int64_t)gj * p.ldc + i0;
-        u32x2 o;
-        if constexpr (OUT == MmaOut::DEQ_BF16) {
-          const float s = p.scale[gj];
-          o[0] = pack_bf16x2(__fmul_rn((float)v[0], s), __fmul_rn((float)v[1], s));
-          o[1] = pack_bf16x2(__fmul_rn((float)v[2], s), __fmul_rn((float)v[3], s));
-        } else if (p.beta == 0.0f) {
-          o[0] = Epi<OUT>::pack(__fmul_rn(p.alpha, v[0]), __fmul_rn(p.alpha, v[1]));
-          o[1] = Epi<OUT>::pack(__fmul_rn(p.alpha, v[2]), __fmul_rn(p.alpha, v[3]));
-        } else {
-          const u32x2 old = *(const u32x2*)c;
-          o[0] = Epi<OUT>::pack(Epi<OUT>::apply(p, v[0], (uint16_t)(old[0] & 0xffff)),
-                                Epi<OUT>::apply(p, v[1], (uint16_t)(old[0] >> 16)));
-          o[1] = Epi<OUT>::pack(Epi<OUT>::apply(p, v[2], (uint16_t)(old[1] & 0xffff)),
-                                Epi<OUT>::apply(p, v[3], (uint16_t)(old[1] >> 16)));
-        }
-        *(u32x2*)c = o;
-      } else {
-        store_run<OUT, STREAM>(p, i0, gj, v, 4, false);
-      }
+      store4<OUT, STREAM>(p, i0, gj, v, true);
     }
   cycle_record(p.probe, t0, probe_slot(wave), wave);
+}
+
+// ---------------------------------------------------------------------------
+// TN path, few columns
+// ---------------------------------------------------------------------------
+
+// For TN problems of up to 64 columns (decoding), which stream A once and do
+// little else (4096 x 16 x 16384: 4.3 TB/s of A, two launches of 128x128 tiles
+// and their sum 3.7): a workgroup takes 16*RM rows and all columns (16*RN), its 8
+// waves every 8th stage of 128 bytes of K. Each wave has a ring of NS stages
+// of its own in LDS, filled and read as gemm_tn128's are (8 rows of 128 bytes
+// per DMA instruction: a row's lanes are adjacent, where reading the matrix
+// cores' fragments straight from memory, 16 rows apart lane by lane, ran at a
+// quarter of the rate), and waits for nobody: no barrier in the K loop, and
+// no split-K pass over memory. The waves' partial sums meet in LDS at the end.
+// What bounds it is the loads a CU has in flight, of which B's (from L2) take
+// RN in RM + RN; two stages at two workgroups per CU were as fast as three or
+// four at one.
+template <class Op, MmaOut OUT, int RM, int RN, int NS>
+__global__ __launch_bounds__(512, 1) void gemm_skinny(KParams batch_p) {
+  const KParams p = batch_view(batch_p);
+  constexpr int NW = 8;
+  constexpr int kEntries = RM * RN * 64;
+  static_assert(kEntries <= 64 * NW, "one sum per thread");
+  constexpr int kStageChunks = (RM + RN) * 16 * kChunks;    // 16-byte chunks of a wave's stage
+  constexpr int kIssue = 2 * (RM + RN);                     // DMA instructions of a stage
+  using Acc = typename Op::Acc16;
+  using E = typename Op::Elem;
+  __shared__ __attribute__((aligned(1024))) i32x4 lds[NW][NS][kStageChunks];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row0 = blockIdx.x * 16 * RM;
+  const int lda_b = (int)(p.lda * Op::kElemBytes);
+  const int ldb_b = (int)(p.ldb * Op::kElemBytes);
+  const int kbytes = p.k * Op::kElemBytes;
+  const int ktiles = (kbytes + kFastKBytes - 1) / kFastKBytes;
+  const int rows_a = min(16 * RM, p.m - row0);
+  constexpr uint32_t kOff = 0x80000000u;
+  // Descriptors as gemm_tn128's: rows past m (n) and chunks past K read zero.
+  const i32x4 rsa = rsrc_words(p.a + (int64_t)row0 * lda_b, (rows_a - 1) * lda_b + kbytes);
+  const i32x4 rsb = rsrc_words(p.b, (p.n - 1) * ldb_b + kbytes);
+  // DMA instruction d of a stage: 8 rows of A (d < 2*RM) or B, lane L to row
+  // L/8 at physical chunk L%8, fetching logical chunk (L%8) ^ swz(row).
+  const int lr = lane >> 3, pc = lane & 7;
+  uint32_t base[kIssue];
+  int chunk[kIssue];
+#pragma unroll
+  for (int d = 0; d < kIssue; ++d) {
+    const bool of_a = d < 2 * RM;
+    const int row = 8 * (of_a ? d : d - 2 * RM) + lr;
+    chunk[d] = 16 * (pc ^ swz(row));
+    base[d] = (uint32_t)(row * (of_a ? lda_b : ldb_b) + chunk[d]);
+  }
+  auto dma = [&](int kt, int st) __attribute__((always_inline)) {
+    const int kb = kt * kFastKBytes;
+#pragma unroll
+    for (int d = 0; d < kIssue; ++d) {
+      const uint32_t v = kb + chunk[d] < kbytes ? base[d] + (uint32_t)kb : kOff;
+      const uint32_t l = (uint32_t)(uintptr_t)(lds_ptr_t)&lds[wave][st][64 * d];
+      if (d < 2 * RM)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     :: "s"(l), "v"(v), "s"(rsa) : "memory");
+      else
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     :: "s"(l), "v"(v), "s"(rsb) : "memory");
+    }
+  };
+
+  const int r16 = lane & 15, q = lane >> 4;
+  // Chunks of a 64-byte k-step to the four 16-lane groups in the order 0, 2,
+  // 1, 3 (A and B alike), as in gemm_tn128: conflict-free reads.
+  const int kq = ((lane >> 3) & 2) | ((lane >> 5) & 1);
+  Acc acc[RM][RN];
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int j = 0; j < RN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0;
+  // Stages wave, wave + NW, ...; one past K is a zero fill, so every wait
+  // counts NS - 1 stages of kIssue loads.
+#pragma unroll
+  for (int s = 0; s < NS; ++s) dma(wave + s * NW, s);
+  int st = 0;
+  for (int kt = wave; kt < ktiles; kt += NW) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * kIssue) : "memory");
+    i32x4 fa[2][RM], fb[2][RN];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int i = 0; i < RM; ++i)
+        fa[ks][i] = lds[wave][st][(16 * i + r16) * kChunks + ((4 * ks + kq) ^ swz(16 * i + r16))];
+#pragma unroll
+      for (int j = 0; j < RN; ++j)
+        fb[ks][j] = lds[wave][st][(16 * (RM + j) + r16) * kChunks + ((4 * ks + kq) ^ swz(16 * j + r16))];
+    }
+    // The fragments are in registers before the stage's slot is filled again.
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    dma(kt + NS * NW, st);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < RM; ++i)
+#pragma unroll
+        for (int j = 0; j < RN; ++j) acc[i][j] = Op::mul16(fa[ks][i], fb[ks][j], acc[i][j]);
+    if (++st == NS) st = 0;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the sums take the rings' place
+  __syncthreads();
+  i32x4* part = &lds[0][0][0];                       // [wave][entry]
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int j = 0; j < RN; ++j)
+      part[wave * kEntries + (i * RN + j) * 64 + lane] = __builtin_bit_cast(i32x4, acc[i][j]);
+  __syncthreads();
+  if (tid >= kEntries) return;
+  // The waves' sums in a fixed order, four rows of one column per thread.
+  E v[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    const i32x4 x = part[w * kEntries + tid];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if constexpr (std::is_integral<E>::value) v[r] = (E)((uint32_t)v[r] + (uint32_t)x[r]);
+      else v[r] += from_bits<E>(x[r]);
+    }
+  }
+  const int e = tid >> 6;
+  const int i0 = row0 + 16 * (e / RN) + 4 * q, gj = 16 * (e % RN) + r16;
+  if (i0 < p.m && gj < p.n)
+    store4<OUT, true>(p, i0, gj, v, ((p.ldc * sizeof(typename Epi<OUT>::T)) & 15) == 0 && ((uintptr_t)p.c & 15) == 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1483,18 +1634,39 @@ constexpr int out_bytes() { return (OUT == MmaOut::F32 || OUT == MmaOut::I32) ? 
 // 32-bit buffer offsets within a 256-row panel, and a C whose columns start
 // on 16-byte boundaries (ldc * sizeof(C) % 16 == 0, aligned C), so that a run of 4 (32-bit)
 // or 8 (16-bit) rows of one column is one vector store.
-template <class Op, MmaOut OUT>
-bool tn_ready(const GemmDesc& d) {
+template <class Op>
+bool tn_operands_ready(const GemmDesc& d) {
   constexpr int EB = Op::kElemBytes;
-  constexpr int OB = out_bytes<OUT>();
   return d.ta && !d.tb && d.k > 0 && ((int64_t)d.k * EB) % 16 == 0 &&
          (d.lda * EB) % 16 == 0 && (d.ldb * EB) % 16 == 0 &&
          ((uintptr_t)d.a % 16) == 0 && ((uintptr_t)d.b % 16) == 0 &&
-         (d.ldc * OB) % 16 == 0 && ((uintptr_t)d.c % 16) == 0 &&
          (d.stride_a * EB) % 16 == 0 && (d.stride_b * EB) % 16 == 0 &&
-         (d.stride_c * OB) % 16 == 0 &&
          (int64_t)kFastTile * d.lda * EB < (1ll << 31) &&
          (int64_t)kFastTile * d.ldb * EB < (1ll << 31);
+}
+
+template <class Op, MmaOut OUT>
+bool tn_ready(const GemmDesc& d) {
+  constexpr int OB = out_bytes<OUT>();
+  return tn_operands_ready<Op>(d) && (d.ldc * OB) % 16 == 0 && ((uintptr_t)d.c % 16) == 0 &&
+         (d.stride_c * OB) % 16 == 0;
+}
+
+// gemm_skinny: one problem of few columns whose operands lie as the TN
+// kernels read them (C may have any alignment), K long enough to give half of
+// its waves a stage. Up to 32 columns always: us, gemm_skinny / 128x128 tiles
+// (split along K and summed where K is long), bf16: 16384 x 16 x 4096 27.5 /
+// 38.1, 4096 x 16 x 16384 31.4 / 36.1, 4096 x 16 x 4096 8.4 / 14.3, 1856 x 3 x
+// 15616 11.1 / 17.2, 128 x 16 x 1024 3.0 / 10.8, 8192 x 20 x 8192 34.1 / 35.6.
+// Up to 64 columns while B, read once per 16 or 32 rows, stays small beside
+// what that saves: 4096 x 64 x 4096 10.9 / 15.5, 1500 x 50 x 3000 8.7 / 19.2,
+// 16384 x 40 x 1024 10.7 / 12.4, but 4096 x 64 x 16384 47 / 38.8 and 16384 x 64
+// x 4096 42.7 / 41.1.
+template <class Op>
+bool skinny_wanted(const GemmDesc& d) {
+  const int64_t kbytes = (int64_t)d.k * Op::kElemBytes;
+  return d.batch == 1 && !d.probe && d.n <= 64 && kbytes >= 4 * kFastKBytes && tn_operands_ready<Op>(d) &&
+         (d.n <= 32 || (kbytes <= 16384 && d.m * kbytes <= (64ll << 20)));
 }
 
 // Other layouts run the TN kernel behind K-contiguous copies of the operands
@@ -1524,6 +1696,7 @@ struct Plan {
   int64_t ldw = 0;                // partials' leading dimension
   size_t w_bytes = 0;
   bool tn = false;                // the TN kernel runs (directly or on copies)
+  bool skinny = false;            // gemm_skinny runs (on the operands as they are)
   int64_t split_ns = 0;           // the split's modelled time (fp32 problems of 256+ tiles)
   bool tn128 = false;             // the TN problem runs on 128x128 tiles (gemm_tn128)
   int tn128_stages = 4;           // its LDS ring: 4 stages (one workgroup per CU) or 2 (two)
@@ -1776,6 +1949,14 @@ Plan direct_operands(const GemmDesc& d, Plan t) {
 
 template <class Op, MmaOut OUT>
 Plan make_plan(const GemmDesc& d) {
+  if constexpr (Op::kM16) {
+    if (skinny_wanted<Op>(d)) {
+      Plan t;
+      t.e = d;
+      t.skinny = true;
+      return t;
+    }
+  }
   Plan t = make_plan_core<Op, OUT>(d);
   if (t.tn) return direct_operands<Op>(d, t);
   if (std::is_same<Op, OpF32>::value || d.batch != 1 || d.probe || !d.pad_copies ||
@@ -1865,7 +2046,7 @@ hipError_t run(const GemmDesc& d, hipStream_t s) {
                  "grxblas: gemm %s->%s ta=%d tb=%d m=%d n=%d k=%d batch=%d kernel=%s copy_a=%d "
                  "copy_b=%d split=%d ring=%d staged=%d direct_a=%d direct_b=%d\n",
                  Op::kName, out_name<OUT>(), (int)d.ta, (int)d.tb, d.m, d.n, d.k, d.batch,
-                 t.tn ? (t.tn128 ? "tn128" : "tn256") : "general64", (int)t.copy_a, (int)t.copy_b, t.split,
+                 t.skinny ? "skinny" : t.tn ? (t.tn128 ? "tn128" : "tn256") : "general64", (int)t.copy_a, (int)t.copy_b, t.split,
                  t.tn && t.tn128 ? t.tn128_stages : 0, (int)(t.tn && t.c_staged),
                  (int)(t.tn && t.a_direct), (int)(t.tn && t.b_direct));
   }
@@ -1886,7 +2067,17 @@ hipError_t run(const GemmDesc& d, hipStream_t s) {
   p.sb = g->stride_b * EB;
   p.sc = g->stride_c * out_bytes<OUT>();
 
-  if (t.tn && (t.split > 1 || t.c_staged)) {
+  if (t.skinny) {
+    if constexpr (Op::kM16) {
+      auto go = [&](auto kern, int rows) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)((g->m + rows - 1) / rows)), dim3(512), 0, s, p);
+      };
+      if (g->n <= 16) go(gemm_skinny<Op, OUT, 1, 1, 2>, 16);
+      else if (g->n <= 32) go(gemm_skinny<Op, OUT, 1, 2, 2>, 16);
+      else if (g->m < 8192) go(gemm_skinny<Op, OUT, 1, 4, 1>, 16);
+      else go(gemm_skinny<Op, OUT, 2, 4, 1>, 32);
+    }
+  } else if (t.tn && (t.split > 1 || t.c_staged)) {
     // Slices (or one, for a staged C): raw partials into the workspace, then
     // the epilogue over their sum.
     KParams q = p;
