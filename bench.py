@@ -374,7 +374,7 @@ def prepare_gemm_bf16(blas, M, cpu_seconds):
 
 def prepare_sgemm(blas):
     """grxblasSgemm fp32 4096^3 (N, N, column-major), fp32 matrix-core roofline.
-    The call copies A K-contiguous (transpose_k) and runs the 256x256-tile
+    The call copies A K-contiguous (copy_operands) and runs the 256x256-tile
     kernel; the timed region holds both."""
     M = N = K = 4096
     log("Sgemm 4096^3: generating inputs")

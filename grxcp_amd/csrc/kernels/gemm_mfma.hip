@@ -162,12 +162,16 @@ struct KParams {
 // partials, which the reduction reads back at once, take plain stores.
 // ---------------------------------------------------------------------------
 
-// One 16-byte run of C: streamed (non-temporal) unless STREAM is false, for
-// an output that is read back right away (split-K partials).
+// One 16-byte run of C at any element alignment (one global_store_dwordx4:
+// gfx950 takes it at any address): streamed (non-temporal) unless STREAM is
+// false, for an output that is read back right away (split-K partials).
+typedef uint32_t u32x4e __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2e __attribute__((ext_vector_type(2), aligned(2)));
 template <bool STREAM, class V>
 __device__ __forceinline__ void put16(void* c, V o) {
-  if constexpr (STREAM) __builtin_nontemporal_store(o, (V*)c);
-  else *(V*)c = o;
+  const u32x4e w = __builtin_bit_cast(u32x4, o);
+  if constexpr (STREAM) __builtin_nontemporal_store(w, (u32x4e*)c);
+  else *(u32x4e*)c = w;
 }
 
 template <MmaOut OUT>
@@ -292,8 +296,9 @@ struct Epi<MmaOut::DEQ_BF16> {
   }
 };
 
-// `count` consecutive rows i0.. of column j (j < n). With `vec`, the caller
-// guarantees a run of kRun elements starting at i0 is 16-byte aligned.
+// `count` consecutive rows i0.. of column j (j < n). With `vec`, a run of
+// kRun elements is one vector store (and read, for which beta != 0 needs C's
+// columns on 16 bytes).
 template <MmaOut OUT, bool STREAM = true, class E>
 __device__ __forceinline__ void store_run(const KParams& p, int i0, int j, const E* v, int count,
                                           bool vec) {
@@ -308,8 +313,7 @@ __device__ __forceinline__ void store_run(const KParams& p, int i0, int j, const
 }
 
 // Rows i0 .. i0+3 of column j (i0 < m, j < n, i0 a multiple of 4), each value
-// as Epi<OUT>::put_run rounds it. `vec`: C's columns are 16-byte aligned, so
-// four rows are one 8- or 16-byte store.
+// as Epi<OUT>::put_run rounds it. `vec`: four rows are one 8- or 16-byte store.
 template <MmaOut OUT, bool STREAM, class E>
 __device__ __forceinline__ void store4(const KParams& p, int i0, int j, const E* v, bool vec) {
   using P = Epi<OUT>;
@@ -331,7 +335,7 @@ __device__ __forceinline__ void store4(const KParams& p, int i0, int j, const E*
       o[0] = P::pack(P::apply(p, v[0], (uint16_t)(old[0] & 0xffff)), P::apply(p, v[1], (uint16_t)(old[0] >> 16)));
       o[1] = P::pack(P::apply(p, v[2], (uint16_t)(old[1] & 0xffff)), P::apply(p, v[3], (uint16_t)(old[1] >> 16)));
     }
-    *(u32x2*)c = o;
+    *(u32x2e*)c = o;
   } else {
     store_run<OUT, STREAM>(p, i0, j, v, 4, false);
   }
@@ -1353,7 +1357,8 @@ __global__ __launch_bounds__(512, 1) void gemm_skinny(KParams batch_p) {
   const int e = tid >> 6;
   const int i0 = row0 + 16 * (e / RN) + 4 * q, gj = 16 * (e % RN) + r16;
   if (i0 < p.m && gj < p.n)
-    store4<OUT, true>(p, i0, gj, v, ((p.ldc * sizeof(typename Epi<OUT>::T)) & 15) == 0 && ((uintptr_t)p.c & 15) == 0);
+    store4<OUT, true>(p, i0, gj, v, (p.beta == 0.0f && p.ibeta == 0) ||
+                                        (((p.ldc * sizeof(typename Epi<OUT>::T)) & 15) == 0 && ((uintptr_t)p.c & 15) == 0));
 }
 
 // ---------------------------------------------------------------------------
@@ -1440,46 +1445,85 @@ __global__ __launch_bounds__(256) void gemm_general(KParams batch_p) {
 }
 
 // ---------------------------------------------------------------------------
-// operand transpose (for layouts the TN kernel cannot read directly)
+// operand copies (for layouts the TN kernels cannot read directly)
 // ---------------------------------------------------------------------------
 
-// Y[c + r*ldy] = X[r + c*ldx] for r < R, c < C, elements of EB bytes, with
-// X read only for c < Cin (columns Cin .. C-1 of Y are zeros: K padded to a
-// multiple of 16 bytes); batch blockIdx.z at X + z*sx, Y + z*sy (elements).
-// 64x64-element tiles through LDS: 16-byte loads along r, 16-byte stores
-// along c. C is a multiple of 16/EB, so an output chunk is wholly inside or
-// outside.
+// One operand to copy K-contiguous: Y[c + r*ldy] = op(X)(r, c) for r < R, c <
+// C, with zeros for Cin <= c < C (K padded to a multiple of 16 bytes); batch z
+// at X + z*sx, Y + z*sy (elements). `transpose`: X is stored r-contiguous
+// (X[r + c*ldx]), else c-contiguous (X[c + r*ldx]: re-laid, its K, pitch or
+// base being off 16 bytes). C is a multiple of 16/EB and Y aligned, so an
+// output chunk is wholly inside or outside.
+struct CopyOp {
+  const uint8_t* x;
+  uint8_t* y;
+  int64_t ldx, sx, ldy, sy;
+  int R, C, Cin;
+  int transpose;
+  int tiles_r;   // 64-row tiles (transpose)
+  int blocks;    // workgroups per batch (0: nothing to copy)
+  int batch;
+};
+
+// 16 bytes at any address.
+typedef uint32_t u32x4b __attribute__((ext_vector_type(4), aligned(1)));
+
+// Both operands' copies in one launch, the first a.blocks workgroups A's:
+// 16-byte loads at element alignment along the stored direction, 16-byte
+// stores along c. (f16, A 1999 x 2301 transposed and B 2301 x 1537 re-laid: 16
+// us in two launches with element-wise loads of the odd pitches.) Transposed
+// tiles of 64x64 elements pass through LDS; a re-laid chunk goes one to a
+// thread. Elements in a chunk that the row's end cuts are read one by one.
 template <int EB>
-__global__ __launch_bounds__(256) void transpose_k(const uint8_t* X, int64_t ldx, int64_t sx,
-                                                   uint8_t* Y, int64_t ldy, int64_t sy, int R,
-                                                   int C, int Cin, int vec_in) {
+__global__ __launch_bounds__(256) void copy_operands(CopyOp a, CopyOp b) {
   constexpr int T = 64;
   constexpr int VE = 16 / EB;        // elements per 16-byte chunk
   constexpr int CPS = T / VE;        // chunks per 64-element segment
   constexpr int PITCH = T * EB + 16; // LDS bytes per c-row
+  using U = std::conditional_t<EB == 4, uint32_t, std::conditional_t<EB == 2, uint16_t, uint8_t>>;
   __shared__ __attribute__((aligned(16))) uint8_t tile[T][PITCH];  // [c][r]
-  const int r0 = blockIdx.x * T, c0 = blockIdx.y * T;
-  X += (int64_t)blockIdx.z * sx * EB;
-  Y += (int64_t)blockIdx.z * sy * EB;
+  const bool first = (int)blockIdx.x < a.blocks;
+  const CopyOp& o = first ? a : b;
+  const int blk = first ? blockIdx.x : blockIdx.x - a.blocks;
+  if ((int)blockIdx.y >= o.batch) return;
+  const uint8_t* X = o.x + (int64_t)blockIdx.y * o.sx * EB;
+  uint8_t* Y = o.y + (int64_t)blockIdx.y * o.sy * EB;
+  if (!o.transpose) {
+    const int cpr = o.C / VE;                              // chunks per row
+    const int64_t q = (int64_t)blk * 256 + threadIdx.x;
+    if (q >= (int64_t)o.R * cpr) return;
+    const int r = (int)(q / cpr), c0 = (int)(q % cpr) * VE;
+    const uint8_t* src = X + ((int64_t)r * o.ldx + c0) * EB;
+    u32x4 w;
+    if (c0 + VE <= o.Cin) {
+      w = *(const u32x4b*)src;
+    } else {
+      U e[VE];
+#pragma unroll
+      for (int i = 0; i < VE; ++i) e[i] = c0 + i < o.Cin ? ((const U*)src)[i] : (U)0;
+      __builtin_memcpy(&w, e, 16);
+    }
+    *(u32x4*)(Y + ((int64_t)r * o.ldy + c0) * EB) = w;
+    return;
+  }
+  const int r0 = blk % o.tiles_r * T, c0 = blk / o.tiles_r * T;
   for (int q = threadIdx.x; q < T * CPS; q += 256) {
     const int c = q / CPS, ch = q % CPS;
     const int gc = c0 + c, gr = r0 + ch * VE;
     uint8_t* dst = &tile[c][ch * 16];
-    const uint8_t* src = X + ((int64_t)gc * ldx + gr) * EB;
-    if (vec_in && gc < Cin && gr + VE <= R) {
-      *(u32x4*)dst = *(const u32x4*)src;
+    const uint8_t* src = X + ((int64_t)gc * o.ldx + gr) * EB;
+    if (gc < o.Cin && gr + VE <= o.R) {
+      *(u32x4*)dst = *(const u32x4b*)src;
     } else {
 #pragma unroll
-      for (int e = 0; e < VE; ++e)
-#pragma unroll
-        for (int b = 0; b < EB; ++b) dst[e * EB + b] = (gc < Cin && gr + e < R) ? src[e * EB + b] : 0;
+      for (int e = 0; e < VE; ++e) ((U*)dst)[e] = (gc < o.Cin && gr + e < o.R) ? ((const U*)src)[e] : (U)0;
     }
   }
   __syncthreads();
   for (int q = threadIdx.x; q < T * CPS; q += 256) {
     const int r = q / CPS, ch = q % CPS;
     const int gr = r0 + r, gc = c0 + ch * VE;
-    if (gr >= R || gc >= C) continue;
+    if (gr >= o.R || gc >= o.C) continue;
     u32x4 w;
     if constexpr (EB == 4) {
 #pragma unroll
@@ -1496,70 +1540,15 @@ __global__ __launch_bounds__(256) void transpose_k(const uint8_t* X, int64_t ldx
                ((uint32_t)tile[ch * VE + 4 * h + 2][r] << 16) |
                ((uint32_t)tile[ch * VE + 4 * h + 3][r] << 24);
     }
-    *(u32x4*)(Y + ((int64_t)gr * ldy + gc) * EB) = w;
+    *(u32x4*)(Y + ((int64_t)gr * o.ldy + gc) * EB) = w;
   }
 }
 
+// Workgroups that copy op(X) (R rows of K): 64x64 tiles, or 256 chunks each.
 template <int EB>
-hipError_t launch_transpose(const void* x, int64_t ldx, int64_t sx, void* y, int64_t ldy,
-                            int64_t sy, int R, int C, int Cin, int batch, hipStream_t s) {
-  const int vec_in = ((uintptr_t)x % 16 == 0) && (ldx * EB) % 16 == 0 && (sx * EB) % 16 == 0;
-  const dim3 grid((unsigned)((R + 63) / 64), (unsigned)((C + 63) / 64), (unsigned)batch);
-  hipLaunchKernelGGL((transpose_k<EB>), grid, dim3(256), 0, s, (const uint8_t*)x, ldx, sx,
-                     (uint8_t*)y, ldy, sy, R, C, Cin, vec_in);
-  return hipGetLastError();
-}
-
-// Y[c + r*ldy] = X[c + r*ldx] for r < R, c < Cin, zeros for Cin <= c < C
-// (C a multiple of 16/EB): an operand that is already K-contiguous but whose
-// K, leading dimension or base the TN kernels cannot take, re-laid in rows of
-// C elements (K padded to 16 bytes). One 16-byte output chunk per thread; a
-// chunk wholly inside the row reads the aligned dwords that hold its 16
-// bytes (four, or five when the source is not 4-byte aligned) and shifts
-// them into place with v_alignbyte; every dword read holds at least one of
-// the chunk's own bytes, so none can fall outside the source's mapped pages.
-// The row's last, partial chunk is read element by element. Batch
-// blockIdx.y at X + z*sx, Y + z*sy (elements).
-template <int EB>
-__global__ __launch_bounds__(256) void repitch_k(const uint8_t* X, int64_t ldx, int64_t sx,
-                                                 uint8_t* Y, int64_t ldy, int64_t sy, int R,
-                                                 int C, int Cin) {
-  constexpr int VE = 16 / EB;
-  const int cpr = C / VE;                                  // chunks per row
-  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (q >= (int64_t)R * cpr) return;
-  const int r = (int)(q / cpr), c0 = (int)(q % cpr) * VE;
-  const uint8_t* src = X + ((int64_t)blockIdx.y * sx + (int64_t)r * ldx + c0) * EB;
-  u32x4 o;
-  if (c0 + VE <= Cin) {
-    const uintptr_t a = (uintptr_t)src;
-    const uint32_t sh = (uint32_t)(a & 3);
-    const uint32_t* w = (const uint32_t*)(a - sh);
-    uint32_t d[5];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) d[i] = w[i];
-    d[4] = sh ? w[4] : 0u;                   // the dword holding byte a+15 when unaligned
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = __builtin_amdgcn_alignbyte(d[i + 1], d[i], sh);
-  } else {
-    uint8_t w[16];
-#pragma unroll
-    for (int e = 0; e < VE; ++e)
-#pragma unroll
-      for (int b = 0; b < EB; ++b) w[e * EB + b] = c0 + e < Cin ? src[e * EB + b] : 0;
-    o = *(const u32x4*)w;
-  }
-  *(u32x4*)(Y + ((int64_t)blockIdx.y * sy + (int64_t)r * ldy + c0) * EB) = o;
-}
-
-template <int EB>
-hipError_t launch_repitch(const void* x, int64_t ldx, int64_t sx, void* y, int64_t ldy, int64_t sy,
-                          int R, int C, int Cin, int batch, hipStream_t s) {
-  const int64_t chunks = (int64_t)R * (C / (16 / EB));
-  const dim3 grid((unsigned)((chunks + 255) / 256), (unsigned)batch);
-  hipLaunchKernelGGL((repitch_k<EB>), grid, dim3(256), 0, s, (const uint8_t*)x, ldx, sx,
-                     (uint8_t*)y, ldy, sy, R, C, Cin);
-  return hipGetLastError();
+int64_t copy_blocks(const CopyOp& o) {
+  if (o.transpose) return (int64_t)o.tiles_r * ((o.C + 63) / 64);
+  return ((int64_t)o.R * (o.C / (16 / EB)) + 255) / 256;
 }
 
 // ---------------------------------------------------------------------------
@@ -1615,9 +1604,10 @@ __global__ __launch_bounds__(256) void reduce_splits(KParams p, const E* ws, int
     for (int h = 0; h < H; ++h) w[h] = *(const i32x4*)(src + z * sstride + 4 * h);
     add(w);
   }
-  // Runs of C are 16-byte aligned unless C is staged (ldc or base off 16 bytes).
+  // Runs of C are 16-byte aligned unless ldc or its base is off 16 bytes.
   using T = typename Epi<OUT>::T;
-  store_run<OUT>(p, i0, j, v, R, ((uintptr_t)((T*)p.c + (int64_t)j * p.ldc + i0) & 15) == 0);
+  store_run<OUT>(p, i0, j, v, R, (p.beta == 0.0f && p.ibeta == 0) ||
+                                     ((uintptr_t)((T*)p.c + (int64_t)j * p.ldc + i0) & 15) == 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1631,9 +1621,10 @@ constexpr int out_bytes() { return (OUT == MmaOut::F32 || OUT == MmaOut::I32) ? 
 
 // The TN kernel's requirements: K-contiguous operands whose rows start on
 // 16-byte boundaries (so every staged chunk is one aligned 16-byte load),
-// 32-bit buffer offsets within a 256-row panel, and a C whose columns start
-// on 16-byte boundaries (ldc * sizeof(C) % 16 == 0, aligned C), so that a run of 4 (32-bit)
-// or 8 (16-bit) rows of one column is one vector store.
+// 32-bit buffer offsets within a 256-row panel; and, where C is read (beta)
+// or dequantised, a C whose columns start on 16-byte boundaries (ldc *
+// sizeof(C) % 16 == 0, aligned C), so that a run of 4 (32-bit) or 8 (16-bit)
+// rows of one column is one aligned access.
 template <class Op>
 bool tn_operands_ready(const GemmDesc& d) {
   constexpr int EB = Op::kElemBytes;
@@ -1645,11 +1636,18 @@ bool tn_operands_ready(const GemmDesc& d) {
          (int64_t)kFastTile * d.ldb * EB < (1ll << 31);
 }
 
+template <MmaOut OUT>
+bool c_ready(const GemmDesc& d) {
+  constexpr int OB = out_bytes<OUT>();
+  return (d.ldc * OB) % 16 == 0 && ((uintptr_t)d.c % 16) == 0 && (d.stride_c * OB) % 16 == 0;
+}
+
+// C off 16-byte boundaries: written in place at element alignment where C is
+// not read (beta = 0), else through the workspace (make_plan).
 template <class Op, MmaOut OUT>
 bool tn_ready(const GemmDesc& d) {
-  constexpr int OB = out_bytes<OUT>();
-  return tn_operands_ready<Op>(d) && (d.ldc * OB) % 16 == 0 && ((uintptr_t)d.c % 16) == 0 &&
-         (d.stride_c * OB) % 16 == 0;
+  const bool c_written = OUT != MmaOut::DEQ_BF16 && d.beta == 0.0f && d.ibeta == 0;
+  return tn_operands_ready<Op>(d) && (c_written || c_ready<OUT>(d));
 }
 
 // gemm_skinny: one problem of few columns whose operands lie as the TN
@@ -1757,7 +1755,7 @@ Plan make_plan_core(const GemmDesc& d) {
     // bytes, the pad zero in both (so every padded product is an exact
     // zero), then the TN kernels on K' (4096^2 x 4095 bf16: 47 TFLOP/s on
     // the 64x64 general kernel). An operand stored K-contiguous is re-laid
-    // row by row (repitch_k), the other transposed (transpose_k).
+    // row by row, the other transposed (copy_operands).
     constexpr int VE = 16 / EB;
     const int kp = (d.k + VE - 1) / VE * VE;
     Plan c = t;
@@ -1886,18 +1884,14 @@ Plan make_plan_core(const GemmDesc& d) {
   return t;
 }
 
-// C whose leading dimension, base or batch stride is not on 16 bytes, which
-// the TN kernels' stores need (bf16 C with m = 4095, or ldc = 500): 16-bit
-// and int8 problems of one batch above the copy threshold keep the TN plan
-// they would have with C aligned, their K loop writing raw partials (one
-// slice, or the plan's split) to the workspace, and reduce_splits applies
-// alpha, beta and the conversion into C, run by run.
-template <MmaOut OUT>
-bool c_ready(const GemmDesc& d) {
-  constexpr int OB = out_bytes<OUT>();
-  return (d.ldc * OB) % 16 == 0 && ((uintptr_t)d.c % 16) == 0 && (d.stride_c * OB) % 16 == 0;
-}
-
+// C whose leading dimension or base is not on 16 bytes (bf16 C with m = 4095,
+// or ldc = 500) and is read (beta != 0) or dequantised: 16-bit and int8
+// problems of one batch above the copy threshold keep the TN plan they would
+// have with C aligned, their K loop writing raw partials (one slice, or the
+// plan's split) to the workspace, and reduce_splits applies alpha, beta and
+// the conversion into C, run by run (make_plan). With beta = 0 the kernels
+// store such a C themselves.
+//
 // A 16-bit op(A) = A (transa N, M-contiguous) or op(B) = B^T (transb T,
 // N-contiguous) on gemm_tn128 (one pass, its K slices, or a staged C) is
 // read where it lies, through
@@ -2018,27 +2012,32 @@ hipError_t run(const GemmDesc& d, hipStream_t s) {
     t.tn = tn_ready<Op, OUT>(d);
   }
   uint8_t* ws = (uint8_t*)d.ws;
-  if (t.copy_a) {
-    // op(A) as rows of kp: A (m x k, m contiguous) transposed, or A^T (rows
-    // of k) re-laid; columns k .. kp-1 zero
-    const hipError_t e =
-        d.ta ? launch_repitch<EB>(d.a, d.lda, d.stride_a, ws, t.kp, (int64_t)d.m * t.kp, d.m, t.kp,
-                                  d.k, t.batch_a, s)
-             : launch_transpose<EB>(d.a, d.lda, d.stride_a, ws, t.kp, (int64_t)d.m * t.kp, d.m,
-                                    t.kp, d.k, t.batch_a, s);
+  if (t.copy_a || t.copy_b) {
+    // op(A) as rows of kp, op(B) as rows of kp per column; columns k .. kp-1 zero
+    auto op = [&](bool wanted, const void* x, bool transpose, int64_t ld, int64_t stride, int rows,
+                  int batch, uint8_t* y) {
+      CopyOp o{};
+      if (!wanted) return o;
+      o.x = (const uint8_t*)x;
+      o.y = y;
+      o.ldx = ld; o.sx = stride;
+      o.ldy = t.kp; o.sy = (int64_t)rows * t.kp;
+      o.R = rows; o.C = t.kp; o.Cin = d.k;
+      o.transpose = transpose;
+      o.tiles_r = (rows + 63) / 64;
+      o.batch = batch;
+      o.blocks = (int)std::min<int64_t>(copy_blocks<EB>(o), 1 << 30);
+      return o;
+    };
+    const CopyOp a = op(t.copy_a, d.a, !d.ta, d.lda, d.stride_a, d.m, t.batch_a, ws);
+    const CopyOp b = op(t.copy_b, d.b, d.tb, d.ldb, d.stride_b, d.n, t.batch_b, ws + t.a_bytes);
+    if (a.blocks == 1 << 30 || b.blocks == 1 << 30) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((copy_operands<EB>), dim3((unsigned)(a.blocks + b.blocks), (unsigned)std::max(a.batch, b.batch)),
+                       dim3(256), 0, s, a, b);
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    t.e.a = ws;
-  }
-  if (t.copy_b) {
-    // op(B) as rows of kp per column j: B (k x n, k contiguous) re-laid, or
-    // B^T (n contiguous) transposed
-    const hipError_t e =
-        !d.tb ? launch_repitch<EB>(d.b, d.ldb, d.stride_b, ws + t.a_bytes, t.kp, (int64_t)d.n * t.kp,
-                                   d.n, t.kp, d.k, t.batch_b, s)
-              : launch_transpose<EB>(d.b, d.ldb, d.stride_b, ws + t.a_bytes, t.kp,
-                                     (int64_t)d.n * t.kp, d.n, t.kp, d.k, t.batch_b, s);
-    if (e != hipSuccess) return e;
-    t.e.b = ws + t.a_bytes;
+    if (t.copy_a) t.e.a = a.y;
+    if (t.copy_b) t.e.b = b.y;
   }
   const GemmDesc* g = &t.e;
   if (log_plans()) {
