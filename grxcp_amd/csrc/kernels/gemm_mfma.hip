@@ -16,10 +16,10 @@
 //    k is masked per 16-byte chunk, so k only has to be a multiple of 16 bytes.
 //
 //  * gemm_general: every transpose combination, any m/n/k, any leading
-//    dimension and alignment. 64x64 tiles, element-wise guarded staging into
-//    LDS in the same [row][k] layout the matrix cores read, 4 waves of one
-//    32x32 MFMA tile each. This is the path the reference's ragged and
-//    transposed gate cases exercise.
+//    dimension and alignment. 64x64 tiles, 16-byte loads at any alignment
+//    staged into LDS in the same [row][k] layout the matrix cores read, 4
+//    waves of one 32x32 MFMA tile each, up to 4 such groups along K. This is
+//    the path the reference's ragged and transposed gate cases exercise.
 //
 // Both kernels are byte-generic: every matrix-core step consumes 16 bytes of
 // A and 16 bytes of B per lane (8 bf16/fp16 or 16 int8 in one v_mfma, 4 fp32
@@ -167,6 +167,7 @@ struct KParams {
 // false, for an output that is read back right away (split-K partials).
 typedef uint32_t u32x4e __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32x2e __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t u32x4b __attribute__((ext_vector_type(4), aligned(1)));   // 16 bytes at any address
 template <bool STREAM, class V>
 __device__ __forceinline__ void put16(void* c, V o) {
   const u32x4e w = __builtin_bit_cast(u32x4, o);
@@ -353,8 +354,8 @@ __device__ __forceinline__ void store_acc_tile(const KParams& p, const typename 
   for (int g = 0; g < 4; ++g) {
     const int i0 = base_i + 8 * g + 4 * (lane >> 5);
     if (i0 >= p.m) continue;
-    E v[4] = {(E)acc[4 * g + 0], (E)acc[4 * g + 1], (E)acc[4 * g + 2], (E)acc[4 * g + 3]};
-    store_run<OUT>(p, i0, j, v, 4, false);
+    const E v[4] = {(E)acc[4 * g + 0], (E)acc[4 * g + 1], (E)acc[4 * g + 2], (E)acc[4 * g + 3]};
+    store4<OUT, true>(p, i0, j, v, p.beta == 0.0f && p.ibeta == 0);
   }
 }
 
@@ -1366,80 +1367,168 @@ __global__ __launch_bounds__(512, 1) void gemm_skinny(KParams batch_p) {
 // ---------------------------------------------------------------------------
 
 constexpr int kGenTile = 64;
-constexpr int kGenKBytes = 64;                 // two MFMA k-steps per stage
-constexpr int kGenRowBytes = kGenKBytes + 16;  // padded row: conflict-free b128 reads
 
-template <class Op, MmaOut OUT>
-__global__ __launch_bounds__(256) void gemm_general(KParams batch_p) {
+// A chunk moved `bytes` >= 0 towards its start, zeros behind it.
+__device__ __forceinline__ u32x4 shift_down(u32x4 w, int bytes) {
+  typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+  u64x2 v = __builtin_bit_cast(u64x2, w);
+  if (bytes >= 8) {
+    v[0] = v[1];
+    v[1] = 0;
+    bytes -= 8;
+  }
+  const int s = 8 * min(bytes, 7);   // two steps: neither shift reaches 64
+  v[0] = bytes >= 8 ? 0 : (v[0] >> s) | (v[1] << 8 << (56 - s));
+  v[1] = bytes >= 8 ? 0 : v[1] >> s;
+  return __builtin_bit_cast(u32x4, v);
+}
+
+// Every transpose combination, shape, leading dimension and alignment: 64x64
+// tiles, one 32x32 MFMA tile per wave, 128-byte stages of K double-buffered in
+// LDS in gemm_tn_fast's swizzled [row][k] layout. A thread stages two 16-byte
+// chunks per operand, loaded at element alignment along the stored direction
+// while the stage before is multiplied: K-contiguous ones land as they are,
+// M- (N-) contiguous ones are spread over their rows, which the swizzle puts
+// on distinct banks. In the last stage of K and in C's edge tiles a chunk that
+// would pass the end of its row (column) is the last 16 bytes that lie inside,
+// shifted to their place with zeros behind: one load and no branches. TINY: an
+// operand's stored rows are shorter than 16 bytes, so elements are loaded one
+// by one. Bound by the latency of a stage's loads (about 2 us for a workgroup
+// alone on its CU), not by a rate, so KG K groups of 4 waves each take every
+// KG-th stage and add their sums in LDS (general_groups).
+// f16, KG as dispatched, against one unpipelined stage of element loads per
+// 64 bytes of K: N,N 256^3 22.0 -> 5.5 us; N,T 300x301x299 26.6 -> 6.9;
+// T,T 128x128x2000 151 -> 14.2; N,N 128x500x500 x 64 160 -> 26.3.
+template <class Op, MmaOut OUT, int KG, bool TINY>
+__global__ __launch_bounds__(256 * KG) void gemm_general(KParams batch_p) {
   const KParams p = batch_view(batch_p);
-  constexpr int EB = Op::kElemBytes;
+  constexpr int EB = Op::kElemBytes, VE = 16 / EB;
+  constexpr int KT = kFastKBytes / EB;         // elements of K per stage
+  constexpr int CPK = kGenTile / VE;           // chunks per k of an M-contiguous operand
   using U = std::conditional_t<EB == 4, uint32_t, std::conditional_t<EB == 2, uint16_t, uint8_t>>;
-  constexpr int KT = kGenKBytes / EB;  // elements of K per stage
-  __shared__ __attribute__((aligned(16))) uint8_t sa[kGenTile * kGenRowBytes];
-  __shared__ __attribute__((aligned(16))) uint8_t sb[kGenTile * kGenRowBytes];
-
+  __shared__ __attribute__((aligned(16))) i32x4 lds[KG][2][2][kGenTile * kChunks];   // [group][operand][buffer]
   const uint64_t t0 = p.probe ? cycle_now() : 0;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int tm = blockIdx.x % p.tiles_m;
-  const int tn = blockIdx.x / p.tiles_m;
-  const int row0 = tm * kGenTile;
-  const int col0 = tn * kGenTile;
+  const int kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const int tid = threadIdx.x & 255, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tm = blockIdx.x % p.tiles_m, tn = blockIdx.x / p.tiles_m;
+  const int row0 = tm * kGenTile, col0 = tn * kGenTile;
+  const bool ca = p.ta, cb = !p.tb;            // K-contiguous
+
+  // An operand: element (r, k) at x + (contiguous ? r*ld + k : k*ld + r).
+  struct Side {
+    const U* x;
+    int64_t ld;
+    int r0, rows;
+    bool kc;
+  };
+  const Side sa{(const U*)p.a, p.lda, row0, p.m, ca}, sb{(const U*)p.b, p.ldb, col0, p.n, cb};
+  const bool interior = row0 + kGenTile <= p.m && col0 + kGenTile <= p.n;
+  u32x4 ra[2], rb[2];
+  // Chunk q of a stage: row q/8, k chunk q%8; or k q/CPK, rows VE*(q%CPK) on.
+  auto load_side = [&](const Side& o, int k0, bool full, u32x4 (&out)[2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int q = tid + 256 * h;
+      const int r = o.r0 + (o.kc ? q / kChunks : VE * (q % CPK));
+      const int k = k0 + (o.kc ? VE * (q % kChunks) : q / CPK);
+      if (full) {
+        out[h] = *(const u32x4b*)(o.x + (o.kc ? r * o.ld + k : k * o.ld + r));
+      } else if constexpr (TINY) {
+        U e[VE];
+#pragma unroll
+        for (int i = 0; i < VE; ++i) {
+          const int ri = o.kc ? r : r + i, ki = o.kc ? k + i : k;
+          e[i] = ri < o.rows && ki < p.k ? o.x[o.kc ? ri * o.ld + ki : ki * o.ld + ri] : (U)0;
+        }
+        __builtin_memcpy(&out[h], e, 16);
+      } else {
+        // The last 16 bytes of the row (column) that start no later than this
+        // chunk, moved down to its place.
+        const int line = o.kc ? min(r, o.rows - 1) : min(k, p.k - 1);
+        const int at = o.kc ? k : r, end = o.kc ? p.k : o.rows;
+        const int from = min(at, end - VE);
+        const u32x4 w = *(const u32x4b*)(o.x + (line * o.ld + from));
+        out[h] = shift_down(w, !o.kc && k >= p.k ? 16 : EB * (at - from));
+      }
+    }
+  };
+  auto load = [&](int k0) __attribute__((always_inline)) {
+    const bool full = interior && k0 + KT <= p.k;
+    load_side(sa, k0, full, ra);
+    load_side(sb, k0, full, rb);
+  };
+  auto store_side = [&](bool kc, i32x4* dst, const u32x4 (&in)[2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int q = tid + 256 * h;
+      if (kc) {
+        const int r = q / kChunks;
+        dst[r * kChunks + ((q % kChunks) ^ swz(r))] = __builtin_bit_cast(i32x4, in[h]);
+      } else {
+        const int k = q / CPK, r = VE * (q % CPK);
+        U e[VE];
+        __builtin_memcpy(e, &in[h], 16);
+#pragma unroll
+        for (int i = 0; i < VE; ++i)
+          ((U*)&dst[(r + i) * kChunks + ((k / VE) ^ swz(r + i))])[k % VE] = e[i];
+      }
+    }
+  };
+  auto store = [&](int buf) __attribute__((always_inline)) {
+    store_side(ca, lds[kg][0][buf], ra);
+    store_side(cb, lds[kg][1][buf], rb);
+  };
 
   using Acc = typename Op::Acc;
+  using E = typename Op::Elem;
   Acc acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0;
-
   const int wm = wave >> 1, wn = wave & 1;
-  const int ktiles = (p.k + KT - 1) / KT;
-  constexpr int kPerThread = kGenTile * KT / 256;
-
-  for (int kt = 0; kt < ktiles; ++kt) {
-    const int k0 = kt * KT;
-    // Stage op(A)[row0.., k0..] as [row][k] and op(B)[k0.., col0..] as [col][k].
-    // The thread -> element map follows the operand's contiguous dimension so
-    // that global reads coalesce.
-#pragma unroll
-    for (int q = 0; q < kPerThread; ++q) {
-      const int e = tid + 256 * q;
-      int r, kk;
-      if (p.ta) { r = e / KT; kk = e % KT; } else { kk = e / kGenTile; r = e % kGenTile; }
-      const int gi = row0 + r, gk = k0 + kk;
-      uint8_t* dst = sa + r * kGenRowBytes + kk * EB;
-      if (gi < p.m && gk < p.k) {
-        const int64_t off = p.ta ? ((int64_t)gi * p.lda + gk) : ((int64_t)gk * p.lda + gi);
-        *(U*)dst = ((const U*)p.a)[off];
-      } else {
-        *(U*)dst = 0;
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < kPerThread; ++q) {
-      const int e = tid + 256 * q;
-      int c, kk;
-      if (!p.tb) { c = e / KT; kk = e % KT; } else { kk = e / kGenTile; c = e % kGenTile; }
-      const int gj = col0 + c, gk = k0 + kk;
-      uint8_t* dst = sb + c * kGenRowBytes + kk * EB;
-      if (gj < p.n && gk < p.k) {
-        const int64_t off = p.tb ? ((int64_t)gk * p.ldb + gj) : ((int64_t)gj * p.ldb + gk);
-        *(U*)dst = ((const U*)p.b)[off];
-      } else {
-        *(U*)dst = 0;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int ks = 0; ks < kGenKBytes / 32; ++ks) {
-      const int kb = ks * 32 + (lane >> 5) * 16;
-      const i32x4 fa = *(const i32x4*)(sa + (wm * 32 + (lane & 31)) * kGenRowBytes + kb);
-      const i32x4 fb = *(const i32x4*)(sb + (wn * 32 + (lane & 31)) * kGenRowBytes + kb);
-      acc = Op::mma(fa, fb, acc);
-    }
-    __syncthreads();
+  const int ar = wm * 32 + (lane & 31), br = wn * 32 + (lane & 31), hh = lane >> 5;
+  if (kg * KT < p.k) {
+    load(kg * KT);
+    store(0);
   }
-
+  __syncthreads();
+  int buf = 0;
+  for (int kb = 0; kb < p.k; kb += KG * KT) {
+    const int k0 = kb + kg * KT;
+    const bool more = k0 + KG * KT < p.k;
+    if (more) load(k0 + KG * KT);
+    if (k0 < p.k) {
+#pragma unroll
+      for (int c = 0; c < kChunks; c += 2) {
+        const i32x4 fa = lds[kg][0][buf][ar * kChunks + ((c + hh) ^ swz(ar))];
+        const i32x4 fb = lds[kg][1][buf][br * kChunks + ((c + hh) ^ swz(br))];
+        acc = Op::mma(fa, fb, acc);
+      }
+    }
+    if (more) store(buf ^ 1);
+    __syncthreads();
+    buf ^= 1;
+  }
+  if constexpr (KG > 1) {
+    // The groups' sums, pairwise, in group 0.
+    int* red = (int*)&lds[0][0][0][0];
+#pragma unroll
+    for (int half = KG / 2; half >= 1; half /= 2) {
+      if (kg >= half && kg < 2 * half)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) red[((kg - half) * 16 + r) * 256 + tid] = bits_of((E)acc[r]);
+      __syncthreads();
+      if (kg < half)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int x = red[(kg * 16 + r) * 256 + tid];
+          if constexpr (std::is_integral<E>::value) acc[r] = (E)((uint32_t)acc[r] + (uint32_t)x);
+          else acc[r] += from_bits<E>(x);
+        }
+      if (half > 1) __syncthreads();
+    }
+    if (kg) return;
+  }
   store_acc_tile<Op, OUT>(p, acc, row0 + wm * 32, col0 + wn * 32, lane);
   cycle_record(p.probe, t0, probe_slot(wave), wave);
 }
@@ -1464,9 +1553,6 @@ struct CopyOp {
   int blocks;    // workgroups per batch (0: nothing to copy)
   int batch;
 };
-
-// 16 bytes at any address.
-typedef uint32_t u32x4b __attribute__((ext_vector_type(4), aligned(1)));
 
 // Both operands' copies in one launch, the first a.blocks workgroups A's:
 // 16-byte loads at element alignment along the stored direction, 16-byte
@@ -1614,7 +1700,9 @@ __global__ __launch_bounds__(256) void reduce_splits(KParams p, const E* ws, int
 // dispatch
 // ---------------------------------------------------------------------------
 
-constexpr int64_t kTransposeMinWork = 1ll << 25;  // m*n*k below this: general path
+// m*n*k below this: the general path as the operands lie; from here on copies
+// for the TN kernels where general_beats_copies does not say otherwise.
+constexpr int64_t kTransposeMinWork = 1ll << 25;
 
 template <MmaOut OUT>
 constexpr int out_bytes() { return (OUT == MmaOut::F32 || OUT == MmaOut::I32) ? 4 : 2; }
@@ -1753,8 +1841,8 @@ Plan make_plan_core(const GemmDesc& d) {
     // K not a multiple of 16 bytes, or the K-contiguous operand unaligned:
     // both operands copied K-contiguous into rows of K rounded up to 16
     // bytes, the pad zero in both (so every padded product is an exact
-    // zero), then the TN kernels on K' (4096^2 x 4095 bf16: 47 TFLOP/s on
-    // the 64x64 general kernel). An operand stored K-contiguous is re-laid
+    // zero), then the TN kernels on K' (the general kernel runs small ones,
+    // general_beats_copies). An operand stored K-contiguous is re-laid
     // row by row, the other transposed (copy_operands).
     constexpr int VE = 16 / EB;
     const int kp = (d.k + VE - 1) / VE * VE;
@@ -1941,6 +2029,42 @@ Plan direct_operands(const GemmDesc& d, Plan t) {
   return t;
 }
 
+inline int64_t general_blocks(const GemmDesc& d) {
+  return (int64_t)((d.m + kGenTile - 1) / kGenTile) * ((d.n + kGenTile - 1) / kGenTile) * d.batch;
+}
+
+// K groups of gemm_general: as many as keep at most one (4 groups) or two (2)
+// workgroups on a CU, and no more than there are stages. bf16 N,N 128x500x500,
+// with 1 / 2 / 4 groups: 8 members (128 workgroups) 16.6 / 10.7 / 8.5 us, 28
+// (448) 19.4 / 14.3 / 16.9, 64 (1024) 26.7 / 27.2 / 32.4. int8 (whose M-
+// contiguous staging spills with 4 groups) N,T 999x199x611: 11.4 / 8.6 / 13.9.
+template <class Op>
+int general_groups(const GemmDesc& d) {
+  const int64_t blocks = general_blocks(d);
+  const int kt = kFastKBytes / Op::kElemBytes;
+  if (d.k <= kt || blocks > 512) return 1;
+  if (d.k <= 2 * kt || blocks > 256 || Op::kElemBytes == 1) return 2;
+  return 4;
+}
+
+// Where plan t would copy operands for the TN kernels, gemm_general on them as
+// they lie: up to one workgroup per CU, and K up to 6 rounds of its 4 groups
+// (int8: 4 of 2). Copies / general, f16: T,T 1003x1001 of k = 1023 20.0 / 14.0
+// us, 2043 29.1 / 23.6, 4003 36.0 / 42.3; N,N 300x300 of 1531 21.2 / 19.5,
+// 2043 25.1 / 25.0, 3000 27.5 / 35.2; int8 N,N 300x300 of 1023 13.8 / 11.9,
+// 2043 18.1 / 20.3; over 256 workgroups, N,N 1500^3 28.6 / 41.8. With a beta
+// the general kernel reads C element by element, and batches share a
+// broadcast operand's copy: both keep the copies. Copies larger than the
+// allocation-free scratch stay copies, so that what it refuses does not depend
+// on this rule.
+template <class Op>
+bool general_beats_copies(const GemmDesc& d, const Plan& t) {
+  return (t.copy_a || t.copy_b) && d.batch == 1 && !d.probe && d.beta == 0.0f && d.ibeta == 0 &&
+         general_blocks(d) <= 256 &&
+         (int64_t)d.k * Op::kElemBytes <= (Op::kElemBytes == 1 ? 1024 : 3072) &&
+         t.bytes() <= kNoAllocScratchBytes;
+}
+
 template <class Op, MmaOut OUT>
 Plan make_plan(const GemmDesc& d) {
   if constexpr (Op::kM16) {
@@ -1952,7 +2076,15 @@ Plan make_plan(const GemmDesc& d) {
     }
   }
   Plan t = make_plan_core<Op, OUT>(d);
-  if (t.tn) return direct_operands<Op>(d, t);
+  if (t.tn) {
+    t = direct_operands<Op>(d, t);
+    if (!general_beats_copies<Op>(d, t)) return t;
+    t = Plan{};
+    t.e = d;
+    t.e.ws = nullptr;
+    t.e.ws_bytes = 0;
+    return t;
+  }
   if (std::is_same<Op, OpF32>::value || d.batch != 1 || d.probe || !d.pad_copies ||
       d.k <= 0 || (int64_t)d.m * d.n * d.k < kTransposeMinWork || c_ready<OUT>(d))
     return t;
@@ -1973,7 +2105,8 @@ Plan make_plan(const GemmDesc& d) {
     c.ldw = ((int64_t)d.m + 7) / 8 * 8;
     c.w_bytes = round256((size_t)c.ldw * d.n * 4);
   }
-  return direct_operands<Op>(d, c);
+  c = direct_operands<Op>(d, c);
+  return general_beats_copies<Op>(d, c) ? t : c;
 }
 
 // GRXBLAS_LOG set (and not "0"): one line on stderr per GemmEx-family call
@@ -2163,8 +2296,15 @@ hipError_t run(const GemmDesc& d, hipStream_t s) {
     p.tiles_n = (g->n + kGenTile - 1) / kGenTile;
     const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n;
     if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_general<Op, OUT>), dim3((unsigned)blocks, g->batch), dim3(256), 0, s,
-                       p);
+    auto go = [&](auto kern, int groups) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)blocks, g->batch), dim3(256 * groups), 0, s, p);
+    };
+    constexpr int VE = 16 / Op::kElemBytes;
+    const int groups = p.probe ? 1 : general_groups<Op>(*g);
+    if ((g->ta ? g->k : g->m) < VE || (g->tb ? g->n : g->k) < VE) go(gemm_general<Op, OUT, 1, true>, 1);
+    else if (groups == 4) go(gemm_general<Op, OUT, 4, false>, 4);
+    else if (groups == 2) go(gemm_general<Op, OUT, 2, false>, 2);
+    else go(gemm_general<Op, OUT, 1, false>, 1);
   }
   return hipGetLastError();
 }

@@ -23,8 +23,8 @@ BF16, F16, F32, I8, I32 = g.GRX_R_16BF, g.GRX_R_16F, g.GRX_R_32F, g.GRX_R_8I, g.
     (BF16, F32, 1, 0, 4097, 2900, 64, 0, "tn256"),
     (BF16, BF16, 1, 0, 257, 255, 8192, 0, "tn128"),     # K slices, summed into C
     (F16, F32, 0, 0, 1999, 1037, 301, 0, "tn128"),      # both operands copied, K padded
-    (BF16, BF16, 1, 1, 511, 1025, 129, 5, "tn128"),
-    (BF16, BF16, 0, 1, 333, 1029, 333, 0, "tn128"),
+    (BF16, BF16, 1, 1, 1027, 1025, 129, 5, "tn128"),
+    (BF16, BF16, 0, 1, 333, 1029, 333, 0, "general64"),
 ])
 def test_c_off_16_bytes(blas, capfd, it, ot, ta, tb, m, n, k, cpad, kernel):
     res = []
