@@ -1746,13 +1746,14 @@ bool tn_ready(const GemmDesc& d) {
 // 15616 11.1 / 17.2, 128 x 16 x 1024 3.0 / 10.8, 8192 x 20 x 8192 34.1 / 35.6.
 // Up to 64 columns while B, read once per 16 or 32 rows, stays small beside
 // what that saves: 4096 x 64 x 4096 10.9 / 15.5, 1500 x 50 x 3000 8.7 / 19.2,
-// 16384 x 40 x 1024 10.7 / 12.4, but 4096 x 64 x 16384 47 / 38.8 and 16384 x 64
-// x 4096 42.7 / 41.1.
+// 16384 x 40 x 1024 10.7 / 12.4, but 4096 x 64 x 16384 47 / 38.8, 7168 x 48 x
+// 4096 17.5 / 17.0 and 16384 x 64 x 4096 42.7 / 41.1.
 template <class Op>
 bool skinny_wanted(const GemmDesc& d) {
   const int64_t kbytes = (int64_t)d.k * Op::kElemBytes;
   return d.batch == 1 && !d.probe && d.n <= 64 && kbytes >= 4 * kFastKBytes && tn_operands_ready<Op>(d) &&
-         (d.n <= 32 || (kbytes <= 16384 && d.m * kbytes <= (64ll << 20)));
+         (d.n <= 32 ? d.m <= 4096 || kbytes <= (d.n <= 16 || d.m <= 8192 ? 8192 : 4096)
+                    : kbytes <= (d.m <= 4096 ? 16384 : 4096) && d.m * kbytes <= (64ll << 20));
 }
 
 // Other layouts run the TN kernel behind K-contiguous copies of the operands

@@ -41,9 +41,10 @@ def test_skinny_int8_exact(blas, m, n, k):
 
 
 def test_skinny_limits(blas, capfd):
-    """Past 64 columns, below 4 stages of K or with an operand off 16 bytes the
-    other kernels run."""
-    for m, n, k, pad in [(128, 65, 512, 0), (128, 16, 248, 0), (128, 16, 512, 4)]:
+    """Past 64 columns, below 4 stages of K, with an operand off 16 bytes or
+    with many rows of long K the other kernels run."""
+    for m, n, k, pad in [(128, 65, 512, 0), (128, 16, 248, 0), (128, 16, 512, 4), (4104, 9, 4104, 0),
+                         (8200, 17, 2056, 0)]:
         res = []
         plans = logged_plans(capfd, lambda: res.append(
             float_case(blas, BF16, F32, 1, 0, m, n, k, 1.0, 0.0, pad, cpad=0)))
