@@ -672,6 +672,7 @@ __global__ __launch_bounds__(64 * kNW, 1) void attn_split(AParams p) {
 
   // The groups' O, maximum and sum to LDS, over the tiles.
   const float l_tot = half_swap_sum(l_run);
+  wait_vmem_all();   // nothing is in flight here: stated for the check of the generated code
   __syncthreads();
   float* mo = (float*)smem;
 #pragma unroll
