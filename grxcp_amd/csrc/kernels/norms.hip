@@ -287,6 +287,12 @@ hipError_t run_rows(NParams p, hipStream_t s) {
     hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), 0, s, p);
   };
   if (need <= 64) go(norm_wave<T, AL, LAYER, 1>, 64, wgrid, 256);
+  // Unaligned rows too few to keep norm_wave's loads in flight: a workgroup per
+  // row, one chunk per thread. In norm_wave a lane's partial chunks are waited
+  // for one after the other: LayerNorm 1255 x 697 fp32 6.1 -> 4.9 us, bf16
+  // 1255 x 999 6.1 -> 5.2; but fp32 2500 x 477 5.9 -> 7.0, bf16 2500 x 999 7.6
+  // -> 8.2.
+  else if (!AL && need <= 256 && p.rows < 2048) go(norm_block<T, AL, LAYER, 256, 1>, 256, bgrid, 256);
   else if (need <= 128) go(norm_wave<T, AL, LAYER, 2>, 128, wgrid, 256);
   else if (need <= 256) go(norm_wave<T, AL, LAYER, 4>, 256, wgrid, 256);
   else if (need <= 512) go(norm_block<T, AL, LAYER, 256, 2>, 512, bgrid, 256);

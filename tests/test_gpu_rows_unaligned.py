@@ -19,7 +19,7 @@ BF16, F16, F32 = g.GRX_R_16BF, g.GRX_R_16F, g.GRX_R_32F
 
 # (type, rows, hidden): chunks are 8 (16-bit) or 4 (fp32) elements; 64, 256,
 # 512, 1024, 2048, 4096 and 8192 of them end a kernel's range
-SHAPES = [(BF16, 5, 9), (F16, 6, 511), (BF16, 9, 2047), (F16, 3, 2049), (BF16, 4, 4097), (F32, 3, 4095),
+SHAPES = [(BF16, 2050, 999), (F32, 2049, 301), (BF16, 5, 9), (F16, 6, 511), (BF16, 9, 2047), (F16, 3, 2049), (BF16, 4, 4097), (F32, 3, 4095),
           (BF16, 2, 8193), (F32, 2, 8193), (BF16, 2, 16385), (F32, 2, 16383), (F16, 2, 32771),
           (F32, 2, 32001), (BF16, 2, 65531), (F32, 1, 65533), (BF16, 2050, 4099)]
 
