@@ -29,7 +29,9 @@
 //  * softmax in the exp2 domain with the running max m tracked in scaled
 //    units: p = exp2(s*scale*log2e - m). m is only raised when a tile's max
 //    exceeds it by more than 8 (p <= 2^8 otherwise, exact in bf16's relative
-//    precision), so the O rescale (and its 128 multiplies) is rare;
+//    precision), so the O rescale (and its 128 multiplies) is rare. m starts at
+//    the lowest finite float, so that -inf scores have weight 0 whichever tile
+//    they fill, and a row of nothing else has l = 0 and comes out NaN;
 //  * P is packed with v_cvt_pk_bf16_f32 (round to nearest even); O is
 //    divided by the row sum once at the end, rounded once, and leaves
 //    through a per-wave LDS region as whole rows (not 8-byte pieces of 32
@@ -62,6 +64,7 @@ constexpr int kNS = 3;    // K/V tile stages in LDS (96 KB at head dim 128)
 constexpr int kQkAhead = 4;  // K fragments read ahead of the score MFMAs
 static_assert(kNS == 3, "the tile loop below is unrolled for three stages");
 constexpr uint32_t kRsrcWord3 = 0x00020000u;
+constexpr float kLowest = -__FLT_MAX__;   // a row's maximum before its first key
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4* lds_s16x4_t;
@@ -176,6 +179,17 @@ __device__ __forceinline__ float half_swap_max(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
+// A row's new maximum in scaled units, mx * c. From a magnitude on where the
+// product's rounding alone would make exp2(mx * c - m) overflow T, it is rounded
+// up instead: the weights of a group of hugely negative scores (a mask added to
+// them) stay finite, so that group adds 0, not 0 * inf, where others dominate.
+template <AttnType T> __device__ __forceinline__ float scaled_max(float mx, float c) {
+  constexpr float kDeep = T == AttnType::BF16 ? 0x1p31f : 0x1p28f;   // half an ulp: 2^7, 2^4
+  const float m = mx * c;
+  const bool up = fabsf(m) >= kDeep && fmaf(mx, c, -m) > 0.0f;
+  const int bits = __builtin_bit_cast(int, m);
+  return up ? __builtin_bit_cast(float, bits + (m > 0.0f ? 1 : -1)) : m;
+}
 __device__ __forceinline__ float half_swap_sum(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
@@ -289,10 +303,10 @@ __device__ __forceinline__ void attend_tile(const AParams& p, const LanePos& l, 
         mx0 = fmaxf(mx0, s[0][r]);
         mx1 = fmaxf(mx1, s[1][r]);
       }
-      const float mx = half_swap_max(fmaxf(mx0, mx1)) * p.c;
-      const bool raise = mx > m_run + 8.0f;
+      const float mx = half_swap_max(fmaxf(mx0, mx1));
+      const bool raise = fmaf(mx, p.c, -m_run) > 8.0f;
       if (__builtin_amdgcn_ballot_w64(raise)) {
-        const float m_new = raise ? mx : m_run;
+        const float m_new = raise ? scaled_max<T>(mx, p.c) : m_run;
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
         m_run = m_new;
         l_run *= alpha;
@@ -462,7 +476,7 @@ __global__ __launch_bounds__(64 * kNW, 1) void attn_fwd(AParams p) {
   for (int i = 0; i < DT; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o_acc[i][r] = 0.0f;
-  float m_run = -INFINITY;
+  float m_run = kLowest;
   float l_run = 0.0f;
 
   const LanePos lp = lane_pos(lane);
@@ -491,7 +505,7 @@ __global__ __launch_bounds__(64 * kNW, 1) void attn_fwd(AParams p) {
     if (last) {
       // O[q, d] = O^T[d, q] / l for this item; then start the next one.
       const float l_tot = half_swap_sum(l_run);
-      const float inv_l = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+      const float inv_l = 1.0f / l_tot;   // l = 0 (every score -inf): 0 * inf is NaN
       // A lane holds 4-value pieces of its query's row, 16 of them spread
       // over the row; stored as they are, one instruction writes 8 bytes in
       // each of 32 rows. Instead the wave parks the rounded tile in its LDS
@@ -532,7 +546,7 @@ __global__ __launch_bounds__(64 * kNW, 1) void attn_fwd(AParams p) {
       for (int i = 0; i < DT; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o_acc[i][r] = 0.0f;
-      m_run = -INFINITY;
+      m_run = kLowest;
       l_run = 0.0f;
       int nbh = 0, nqt = 0;
       if (item_at(p, map, round + 1, &nbh, &nqt)) {
@@ -653,7 +667,7 @@ __global__ __launch_bounds__(64 * kNW, 1) void attn_split(AParams p) {
   for (int i = 0; i < DT; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o_acc[i][r] = 0.0f;
-  float m_run = -INFINITY, l_run = 0.0f;
+  float m_run = kLowest, l_run = 0.0f;
   landed();
   for (int s = 0; s < steps; ++s) {
     const int st = NS == 2 ? s & 1 : 0;
@@ -713,7 +727,7 @@ __global__ __launch_bounds__(64 * kNW, 1) void attn_split(AParams p) {
         for (int e = 0; e < 4; ++e) o[4 * q + e] = fmaf(scale, v[e], o[4 * q + e]);
       }
     }
-    const float inv_l = l > 0.0f ? 1.0f / l : 0.0f;
+    const float inv_l = 1.0f / l;   // as in attn_fwd
     i32x4 out;
 #pragma unroll
     for (int q = 0; q < 4; ++q) out[q] = (int)IO::pack2(o[2 * q] * inv_l, o[2 * q + 1] * inv_l);

@@ -61,3 +61,35 @@ def test_attention_heads_in_one_block(dnn, H, S, D):
     """39 and 33 causal items on each XCD's 32 workgroups: one block of all
     its heads, dealt in a snake from the heaviest items on."""
     check_heads(dnn, BF16, 1, H, S, D, True)
+
+
+# Keys masked by a bias column of K: a tail, one key, the first tile (left
+# padding); heads and S for 64-query and 128-query items and for attn_fwd.
+MASKS = {"tail64": slice(64, None), "tail128": slice(128, None), "tail256": slice(256, None),
+         "key64": slice(64, 65), "key128": slice(128, 129), "head64": slice(0, 64)}
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("t,fill", [(BF16, -np.inf), (BF16, -3.3895314e38), (BF16, -1e30), (F16, -np.inf),
+                                    (F16, -65504.0)])
+@pytest.mark.parametrize("D,H,S", [(64, 6, 500), (128, 6, 500), (64, 64, 300), (128, 64, 300), (64, 200, 300),
+                                   (128, 200, 300)])
+def test_attention_masked_keys(dnn, D, H, S, t, fill, causal):
+    """Key groups (and a first tile) whose every score is -inf or hugely
+    negative have weight 0; a row that sees only -inf scores is NaN."""
+    r = np.random.default_rng(S + D)
+    q = r.standard_normal((1, H, S, D)).astype(np.float32)
+    k = r.standard_normal((1, H, S, D)).astype(np.float32)
+    q[..., 0] = 1.0
+    names = sorted(MASKS)
+    for h, name in enumerate(names):
+        k[0, h, MASKS[name]] = 0.0
+        k[0, h, MASKS[name], 0] = fill
+    o, qq, kq, v = run_attention(dnn, t, 1, H, S, D, causal, seed=3, q=q, k=k)
+    for h, name in enumerate(names):
+        ref = O.attention_head(qq[0, h], kq[0, h], v[0, h], causal, D ** -0.5)
+        lo = 64 if causal and name == "head64" else 0     # rows before lo see masked keys only
+        if np.isinf(fill):
+            assert np.isnan(o[0, h, :lo]).all()
+        assert np.isfinite(o[0, h, lo:]).all(), name
+        assert normwise_rel_err(o[0, h, lo:], ref[lo:]) <= 1e-2, name
