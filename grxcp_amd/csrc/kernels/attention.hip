@@ -827,9 +827,10 @@ hipError_t run(const AttnDesc& d, hipStream_t s) {
   if ((int64_t)d.B * d.H * p.qtiles > 0x7fffffff) return hipErrorInvalidValue;
   // (a cycle probe's slots are counted for attn_fwd)
   const int qw = d.probe ? 0 : split_blocks((int64_t)d.B * d.H, d.S, D, p.causal);
-  if (qw) {
+  const int64_t items = qw ? (int64_t)p.heads * ((d.S + 32 * qw - 1) / (32 * qw)) : 0;
+  if (qw && items <= max_workgroups(64 * kNW)) {
     p.qtiles = (d.S + 32 * qw - 1) / (32 * qw);
-    const dim3 grid((unsigned)(p.heads * p.qtiles));
+    const dim3 grid((unsigned)items);
     if (qw == 4) hipLaunchKernelGGL((attn_split<T, D, 4, 2>), grid, dim3(64 * kNW), 0, s, p);
     else hipLaunchKernelGGL((attn_split<T, D, 2, D == 64 ? 2 : 1>), grid, dim3(64 * kNW), 0, s, p);
     return hipGetLastError();

@@ -11,6 +11,9 @@
 
 namespace grxk {
 
+// HIP takes fewer than 2^32 threads along a launch's x dimension.
+inline int64_t max_workgroups(int threads) { return 0xffffffffll / threads; }
+
 // Element types the matrix-core GEMM reads and the epilogue it ends in.
 enum class MmaIn { BF16, F16, I8, F32 };   // F32: Sgemm's large problems
 enum class MmaOut {
