@@ -283,6 +283,7 @@ hipError_t run_rows(NParams p, hipStream_t s) {
   // more (its first and last are partial) where a kernel has room for it.
   const int need = nchunks + (AL ? 0 : 1);
   auto go = [&](auto kern, int cap, unsigned grid, int threads) {
+    grid = (unsigned)std::min<int64_t>(grid, max_workgroups(threads));   // the kernels loop over more rows
     p.align_mask = need <= cap ? V - 1 : 0;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), 0, s, p);
   };

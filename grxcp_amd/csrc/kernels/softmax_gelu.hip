@@ -176,7 +176,7 @@ __global__ __launch_bounds__(NT) void softmax_block(RParams p) {
       for (int e = 0; e < V; ++e) o[e] = (T == NormType::F32 ? v[e] : exp_le0<T>(v[e] - mx)) * inv;
       rc.store(yrow, c, IO::pack(o));
     }
-    // Only a grid of fewer workgroups than rows (over 2^30 rows) loops: the
+    // Only a grid of fewer workgroups than rows (max_workgroups) loops: the
     // next row's partials must not land before every wave has read these.
     if (row + gridDim.x < p.rows) __syncthreads();
   }
@@ -359,6 +359,7 @@ hipError_t run_softmax(const RowDesc& d, hipStream_t s) {
   // more (its first and last are partial) where a kernel has room for it.
   const int need = nchunks + (AL ? 0 : 1);
   auto go = [&](auto kern, int cap, unsigned grid, int threads) {
+    grid = (unsigned)std::min<int64_t>(grid, max_workgroups(threads));   // the kernels loop over more rows
     p.align_mask = need <= cap ? V - 1 : 0;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), 0, s, p);
   };

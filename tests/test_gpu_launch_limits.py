@@ -44,3 +44,24 @@ def test_attention_many_heads(gpu, dnn):
         got = dec(o.download(np.uint16, head, offset=2 * head * first), BF16).reshape(S, D)
         assert normwise_rel_err(got, ref) <= 1e-2, first
     o.close()
+
+
+def test_softmax_many_unaligned_rows(gpu, dnn):
+    """2^23 rows of 4105 elements, in place, one to a 512-thread workgroup."""
+    rows, hidden = 1 << 23, 4105
+    x = big_buffer(gpu, rows * hidden * 2)
+    r = np.random.default_rng(1)
+    xe = enc(r.standard_normal((1, hidden)).astype(np.float32), BF16)
+    at = (0, rows // 2, rows - 2, rows - 1)
+    for i in at:
+        x.upload(xe, offset=2 * hidden * i)
+    xd = g.TensorDesc(BF16, [rows, hidden])
+    say("softmax of 2^23 rows")
+    s = dnn.softmax(xd, x.p, xd, x.p)
+    assert s == g.SUCCESS, g.STATUS[s]
+    g.synchronize()
+    ref = O.softmax(dec(xe, BF16).reshape(1, hidden))[0]
+    for i in at:
+        got = dec(x.download(np.uint16, hidden, offset=2 * hidden * i), BF16)
+        assert np.all(np.abs(got - ref) <= 2.0 ** -8 * np.abs(ref)), i
+    x.close()
