@@ -1554,23 +1554,25 @@ struct CopyOp {
   int batch;
 };
 
-// Both operands' copies in one launch, the first a.blocks workgroups A's:
-// 16-byte loads at element alignment along the stored direction, 16-byte
-// stores along c. (f16, A 1999 x 2301 transposed and B 2301 x 1537 re-laid: 16
+// Both operands' copies in one launch, the first a.blocks workgroups A's
+// (block0: of all of them, where one launch cannot take that many): 16-byte
+// loads at element alignment along the stored direction, 16-byte stores along
+// c. (f16, A 1999 x 2301 transposed and B 2301 x 1537 re-laid: 16
 // us in two launches with element-wise loads of the odd pitches.) Transposed
 // tiles of 64x64 elements pass through LDS; a re-laid chunk goes one to a
 // thread. Elements in a chunk that the row's end cuts are read one by one.
 template <int EB>
-__global__ __launch_bounds__(256) void copy_operands(CopyOp a, CopyOp b) {
+__global__ __launch_bounds__(256) void copy_operands(CopyOp a, CopyOp b, int block0) {
   constexpr int T = 64;
   constexpr int VE = 16 / EB;        // elements per 16-byte chunk
   constexpr int CPS = T / VE;        // chunks per 64-element segment
   constexpr int PITCH = T * EB + 16; // LDS bytes per c-row
   using U = std::conditional_t<EB == 4, uint32_t, std::conditional_t<EB == 2, uint16_t, uint8_t>>;
   __shared__ __attribute__((aligned(16))) uint8_t tile[T][PITCH];  // [c][r]
-  const bool first = (int)blockIdx.x < a.blocks;
+  const int block = block0 + (int)blockIdx.x;
+  const bool first = block < a.blocks;
   const CopyOp& o = first ? a : b;
-  const int blk = first ? blockIdx.x : blockIdx.x - a.blocks;
+  const int blk = first ? block : block - a.blocks;
   if ((int)blockIdx.y >= o.batch) return;
   const uint8_t* X = o.x + (int64_t)blockIdx.y * o.sx * EB;
   uint8_t* Y = o.y + (int64_t)blockIdx.y * o.sy * EB;
@@ -2166,10 +2168,14 @@ hipError_t run(const GemmDesc& d, hipStream_t s) {
     const CopyOp a = op(t.copy_a, d.a, !d.ta, d.lda, d.stride_a, d.m, t.batch_a, ws);
     const CopyOp b = op(t.copy_b, d.b, d.tb, d.ldb, d.stride_b, d.n, t.batch_b, ws + t.a_bytes);
     if (a.blocks == 1 << 30 || b.blocks == 1 << 30) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((copy_operands<EB>), dim3((unsigned)(a.blocks + b.blocks), (unsigned)std::max(a.batch, b.batch)),
-                       dim3(256), 0, s, a, b);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    const int64_t blocks = (int64_t)a.blocks + b.blocks;
+    for (int64_t b0 = 0; b0 < blocks; b0 += max_workgroups(256)) {
+      hipLaunchKernelGGL((copy_operands<EB>),
+                         dim3((unsigned)std::min(blocks - b0, max_workgroups(256)), (unsigned)std::max(a.batch, b.batch)),
+                         dim3(256), 0, s, a, b, (int)b0);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+    }
     if (t.copy_a) t.e.a = a.y;
     if (t.copy_b) t.e.b = b.y;
   }
