@@ -1742,20 +1742,31 @@ bool tn_ready(const GemmDesc& d) {
 
 // gemm_skinny: one problem of few columns whose operands lie as the TN
 // kernels read them (C may have any alignment), K long enough to give half of
-// its waves a stage. Up to 32 columns always: us, gemm_skinny / 128x128 tiles
-// (split along K and summed where K is long), bf16: 16384 x 16 x 4096 27.5 /
-// 38.1, 4096 x 16 x 16384 31.4 / 36.1, 4096 x 16 x 4096 8.4 / 14.3, 1856 x 3 x
-// 15616 11.1 / 17.2, 128 x 16 x 1024 3.0 / 10.8, 8192 x 20 x 8192 34.1 / 35.6.
-// Up to 64 columns while B, read once per 16 or 32 rows, stays small beside
-// what that saves: 4096 x 64 x 4096 10.9 / 15.5, 1500 x 50 x 3000 8.7 / 19.2,
-// 16384 x 40 x 1024 10.7 / 12.4, but 4096 x 64 x 16384 47 / 38.8, 7168 x 48 x
-// 4096 17.5 / 17.0 and 16384 x 64 x 4096 42.7 / 41.1.
+// its waves a stage. It splits K over the 8 waves of a workgroup only, so K is
+// bounded: a workgroup's time is the latency of stages / 8 loads, longer the
+// more of a stage is B's columns, while the 128x128 tiles' K slices take about
+// 14 us on any such problem. Columns and the bytes of K where the two meet
+// (up to 3072 rows, A from memory; us, gemm_skinny / 128x128 tiles, bf16): 8
+// columns 28 KB (2048 rows 19 / 19, at 64 KB 47 / 39), 16 columns 24 KB (256
+// rows 16 / 15, at 128 KB 73 / 38), 32 columns 16 KB (1024 rows 15.9 / 16, at
+// 32 KB 26 / 16), 64 columns 10 KB (17 / 17, at 16 KB 21 / 16). With more rows
+// memory bounds both: 4096 x 16, K of 32 KB 32 / 38, of 64 KB 55 / 67, of 80
+// KB 67 / 63; 3584 x 8 of 80 KB 55 / 59; 4096 x 32 of 32 KB 35 / 39, of 40 KB
+// 44 / 38. Past 4096 rows a CU has several workgroups, each reading B again:
+// 16384 x 16 x 4096 27.5 / 38.1, 8192 x 20 x 4096 19.6 / 20 (of 8192 34.1 /
+// 35.6), 12288 x 32 of 4 KB 19 / 20, of 8 KB none gained; 16384 x 40 x 1024
+// 10.7 / 12.4, but 16384 x 64 x 4096 42.7 / 41.1.
 template <class Op>
 bool skinny_wanted(const GemmDesc& d) {
   const int64_t kbytes = (int64_t)d.k * Op::kElemBytes;
-  return d.batch == 1 && !d.probe && d.n <= 64 && kbytes >= 4 * kFastKBytes && tn_operands_ready<Op>(d) &&
-         (d.n <= 32 ? d.m <= 4096 || kbytes <= (d.n <= 16 || d.m <= 8192 ? 8192 : 4096)
-                    : kbytes <= (d.m <= 4096 ? 16384 : 4096) && d.m * kbytes <= (64ll << 20));
+  if (d.batch != 1 || d.probe || d.n > 64 || kbytes < 4 * kFastKBytes || !tn_operands_ready<Op>(d)) return false;
+  if (d.m > 4096)
+    return kbytes <= (d.n <= 16 || (d.n <= 32 && d.m <= 8192) ? 8192 : 4096) &&
+           (d.n <= 32 || d.m * kbytes <= (64ll << 20));
+  if (d.n <= 8) return d.m > 2560 || kbytes <= (28 << 10);
+  if (d.n <= 16) return kbytes <= (d.m > 3072 ? 64 << 10 : 24 << 10);
+  if (d.n <= 32) return kbytes <= (d.m > 3072 ? 32 << 10 : 16 << 10);
+  return kbytes <= (10 << 10);
 }
 
 // Other layouts run the TN kernel behind K-contiguous copies of the operands

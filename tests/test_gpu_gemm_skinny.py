@@ -50,3 +50,17 @@ def test_skinny_limits(blas, capfd):
             float_case(blas, BF16, F32, 1, 0, m, n, k, 1.0, 0.0, pad, cpad=0)))
         assert res == [(0, 0)]
         assert [p["kernel"] for p in plans] != ["skinny"], (m, n, k, pad)
+
+
+@pytest.mark.parametrize("m,n,kmax", [(16, 8, 14336), (2576, 3, 0), (128, 16, 12288), (3088, 32, 16384),
+                                      (128, 17, 8192), (64, 33, 5120), (4096, 64, 5120)])
+def test_skinny_k_bound(blas, capfd, m, n, kmax):
+    """K of the longest that one workgroup takes runs on gemm_skinny, K one
+    16-byte chunk longer on the 128x128 tiles and their K slices (kmax 0: no
+    bound); both exact."""
+    for k in (kmax, kmax + 8) if kmax else (40000,):
+        res = []
+        plans = logged_plans(capfd, lambda: res.append(
+            float_case(blas, BF16, F32, 1, 0, m, n, k, 1.0, 0.0, 0, cpad=0)))
+        assert res == [(0, 0)]
+        assert [p["kernel"] == "skinny" for p in plans] == [k <= kmax or not kmax], (k, plans)
