@@ -22,8 +22,10 @@
 //    LayerNorm's variance is the two-pass (x - mean)^2 form over the cached
 //    registers, which costs no extra memory traffic.
 //  * rows whose length, pitch or base alignment rule out 16-byte boundaries
-//    run the same kernels with chunks at element alignment and a partial last
-//    chunk (AL = false).
+//    run the same kernels: those of a wavefront as whole chunks at element
+//    alignment, of which the last ends with the row (WholeChunks), longer ones
+//    on memory's 16-byte boundaries with a partial first and last chunk
+//    (RowChunks, AL = false).
 
 #include "../launch.h"
 #include "device_common.h"
@@ -86,7 +88,8 @@ __global__ __launch_bounds__(NT) void norm_block(NParams p) {
   // gamma and beta are held beside the row (aligned rows: for all rows of
   // the workgroup; others have their chunks at offsets of their own). With
   // more than 4 chunks per thread the registers hold the row alone, and gamma
-  // and beta are read when they are used.
+  // and beta are read when they are used (16 chunks of fp32, LayerNorm, still
+  // spill 24 registers).
   constexpr bool HOLD = NQ <= 4;
   u32x4 graw[HOLD ? NQ : 1], braw[HOLD ? NQ : 1];
   auto weights = [&](const RowChunks<T, AL>& rc) __attribute__((always_inline)) {
@@ -181,8 +184,13 @@ __global__ __launch_bounds__(NT) void norm_block(NParams p) {
 // One row per 64-lane wavefront, for rows of up to NC x 64 16-byte chunks:
 // the row lives in the wave's registers, both statistics are wave
 // reductions (lane moves only: no LDS, no barrier), so every wave streams
-// independently and a CU keeps ~20 rows of loads in flight.
-template <NormType T, bool AL, bool LAYER, int NC>
+// independently and a CU keeps ~20 rows of loads in flight. Rows off 16-byte
+// boundaries take WholeChunks: with RowChunks a wave waits for its partial
+// chunks one after the other and issues a load per element of them (LayerNorm,
+// us, RowChunks / WholeChunks: bf16 2500 x 697 7.1 / 4.8, 2048 x 999 6.7 / 4.8,
+// 16384 x 2047 56.9 / 28.1, 16384 x 511 20.5 / 9.0; fp32 2500 x 999 7.1 / 5.6,
+// but 8192 x 777 11.6 / 12.7). Only rows shorter than a chunk keep RowChunks.
+template <NormType T, class Chunks, bool LAYER, int NC>
 __global__ __launch_bounds__(256) void norm_wave(NParams p) {
   using IO = Io<T>;
   constexpr int V = IO::kVec;
@@ -193,7 +201,7 @@ __global__ __launch_bounds__(256) void norm_wave(NParams p) {
   for (int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); row < p.rows; row += nwaves) {
     const uint8_t* xrow = p.x + row * p.x_rs * (int64_t)(16 / V);
     uint8_t* yrow = p.y + row * p.y_rs * (int64_t)(16 / V);
-    const RowChunks<T, AL> rc(xrow, p.hidden, p.align_mask);
+    const Chunks rc(xrow, p.hidden, p.align_mask);
     u32x4 raw[NC];
 #pragma unroll
     for (int q = 0; q < NC; ++q) {
@@ -205,7 +213,10 @@ __global__ __launch_bounds__(256) void norm_wave(NParams p) {
       float v[V];
       IO::unpack(raw[q], v);
 #pragma unroll
-      for (int e = 0; e < V; ++e) s += LAYER ? v[e] : v[e] * v[e];
+      for (int e = 0; e < V; ++e) {
+        const float x = !Chunks::kRepeats || rc.has(lane + 64 * q, e) ? v[e] : 0.0f;
+        s += LAYER ? x : x * x;
+      }
     }
     // Keep only the packed row live between passes (unpacking again is a
     // couple of ALU ops; holding 8*NC floats would halve the waves per CU).
@@ -222,7 +233,7 @@ __global__ __launch_bounds__(256) void norm_wave(NParams p) {
         if (!rc.any(c)) continue;
         float v[V];
         IO::unpack(raw[q], v);
-        if (AL || rc.whole(c)) {
+        if (rc.whole(c)) {
 #pragma unroll
           for (int e = 0; e < V; ++e) {
             const float d = v[e] - mean;
@@ -287,15 +298,11 @@ hipError_t run_rows(NParams p, hipStream_t s) {
     p.align_mask = need <= cap ? V - 1 : 0;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), 0, s, p);
   };
-  if (need <= 64) go(norm_wave<T, AL, LAYER, 1>, 64, wgrid, 256);
-  // Unaligned rows too few to keep norm_wave's loads in flight: a workgroup per
-  // row, one chunk per thread. In norm_wave a lane's partial chunks are waited
-  // for one after the other: LayerNorm 1255 x 697 fp32 6.1 -> 4.9 us, bf16
-  // 1255 x 999 6.1 -> 5.2; but fp32 2500 x 477 5.9 -> 7.0, bf16 2500 x 999 7.6
-  // -> 8.2.
-  else if (!AL && need <= 256 && p.rows < 2048) go(norm_block<T, AL, LAYER, 256, 1>, 256, bgrid, 256);
-  else if (need <= 128) go(norm_wave<T, AL, LAYER, 2>, 128, wgrid, 256);
-  else if (need <= 256) go(norm_wave<T, AL, LAYER, 4>, 256, wgrid, 256);
+  using Wave = std::conditional_t<AL, RowChunks<T, true>, WholeChunks<T>>;
+  if (p.hidden < V) go(norm_wave<T, RowChunks<T, AL>, LAYER, 1>, 64, wgrid, 256);
+  else if (nchunks <= 64) go(norm_wave<T, Wave, LAYER, 1>, 64, wgrid, 256);
+  else if (nchunks <= 128) go(norm_wave<T, Wave, LAYER, 2>, 128, wgrid, 256);
+  else if (nchunks <= 256) go(norm_wave<T, Wave, LAYER, 4>, 256, wgrid, 256);
   else if (need <= 512) go(norm_block<T, AL, LAYER, 256, 2>, 512, bgrid, 256);
   else if (need <= 1024) go(norm_block<T, AL, LAYER, 512, 2>, 1024, bgrid, 512);
   else if (need <= 2048) go(norm_block<T, AL, LAYER, 1024, 2>, 2048, bgrid, 1024);

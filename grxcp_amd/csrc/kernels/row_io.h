@@ -87,6 +87,7 @@ typedef uint32_t u32x4e __attribute__((ext_vector_type(4), aligned(2)));
 template <NormType T, bool AL>
 struct RowChunks {
   static constexpr int V = Io<T>::kVec;
+  static constexpr bool kRepeats = false;
   int hidden, head = 0;
   __device__ __forceinline__ RowChunks(const uint8_t* row, int hidden_, int align_mask) : hidden(hidden_) {
     if constexpr (!AL) head = (int)((uintptr_t)row / (16 / V)) & align_mask;
@@ -151,6 +152,31 @@ struct RowChunks {
         else ((uint16_t*)row)[first(c) + e] = (uint16_t)((e & 1) ? w[e >> 1] >> 16 : w[e >> 1]);
       }
     }
+  }
+};
+
+// A row of at least V elements at any element alignment as whole chunks: chunk
+// c starts at element c*V, but the last one ends with the row and repeats
+// elements of the one before it, which `has` leaves to that one (both store the
+// same values). Every load and store is one instruction without a branch.
+template <NormType T>
+struct WholeChunks {
+  static constexpr int V = Io<T>::kVec;
+  static constexpr bool kRepeats = true;
+  int hidden;
+  __device__ __forceinline__ WholeChunks(const uint8_t*, int hidden_, int) : hidden(hidden_) {}
+  __device__ __forceinline__ int first(int c) const { return min(c * V, hidden - V); }
+  __device__ __forceinline__ bool any(int c) const { return c * V < hidden; }
+  __device__ __forceinline__ bool whole(int c) const { return c * V + V <= hidden; }
+  __device__ __forceinline__ bool has(int c, int e) const { return first(c) + e >= c * V; }
+  template <bool STREAM = true>
+  __device__ __forceinline__ u32x4 load(const uint8_t* row, int c, u32x4 none) const {
+    const u32x4e* q = (const u32x4e*)(row + (int64_t)first(c) * (16 / V));
+    if (!any(c)) return none;
+    return STREAM ? __builtin_nontemporal_load(q) : *q;
+  }
+  __device__ __forceinline__ void store(uint8_t* row, int c, u32x4 w) const {
+    if (any(c)) __builtin_nontemporal_store((u32x4e)w, (u32x4e*)(row + (int64_t)first(c) * (16 / V)));
   }
 };
 

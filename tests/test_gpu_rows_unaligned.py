@@ -87,3 +87,43 @@ def test_gelu_contiguous_odd_rows(dnn, t, rows, hidden):
     check(dec(out[:xe.size].copy(), t).reshape(rows, hidden),
           O.gelu(dec(xe, t).reshape(rows, hidden), g.GELU_ERF).reshape(rows, hidden), t,
           atol={BF16: 1e-6, F16: 1e-6, F32: 1e-7}[t])
+
+
+# Lengths around the chunk (shorter rows take a path of their own), one, two
+# and four chunks per lane, and what each leaves for the last chunk.
+@pytest.mark.parametrize("layer", [False, True])
+@pytest.mark.parametrize("t,hidden", [(BF16, h) for h in (1, 7, 8, 9, 15, 511, 512, 513, 1023, 1025, 2041, 2048, 2049)] +
+                         [(F16, h) for h in (3, 10, 505, 1017)] +
+                         [(F32, h) for h in (1, 3, 4, 5, 7, 255, 256, 257, 511, 513, 1021, 1024, 1025)])
+def test_short_unaligned_norms_in_place(dnn, t, hidden, layer):
+    """The last chunk of a row repeats elements of the one before it: they
+    count once in the statistics, and in place no chunk reads what another
+    has already replaced. A NaN among the repeated elements stays in its row."""
+    rows, pitch = 7, hidden + 1
+    r = np.random.default_rng(hidden)
+    x = (1.5 + 2.0 * r.standard_normal((rows, hidden))).astype(np.float32)
+    xe = enc(x, t)
+    ge, be = (enc(a.astype(np.float32), t) for a in (1 + 0.1 * r.standard_normal(hidden), r.standard_normal(hidden)))
+    xe[4, max(0, hidden - 3)] = 0x7FC1 if t == BF16 else 0x7E01 if t == F16 else np.nan
+    poison = np.asarray(0x7FC1 if t != F32 else np.float32(np.nan), nptype(t))
+    buf = np.full(1 + rows * pitch, poison, nptype(t))
+    buf[1:].reshape(rows, pitch)[:, :hidden] = xe
+    dx, dg, db = to_dev(buf), to_dev(np.concatenate([poison[None], ge])), to_dev(np.concatenate([poison[None], be]))
+    xd, wd = g.TensorDesc(t, [rows, hidden], [pitch, 1]), g.TensorDesc(t, [hidden])
+    p, pg, pb = (offset(b, t) for b in (dx, dg, db))
+    say(f"{'layer' if layer else 'rms'}norm t={t} hidden={hidden} in place, one element off")
+    s = dnn.layernorm(xd, p, wd, pg, pb, 1e-6, xd, p) if layer else dnn.rmsnorm(xd, p, wd, pg, 1e-6, xd, p)
+    assert s == g.SUCCESS, g.STATUS[s]
+    g.synchronize()
+    out = dx.download(nptype(t), buf.size)
+    body = out[1:].reshape(rows, pitch)
+    around = np.concatenate([out[:1], body[:, hidden:].reshape(-1)])
+    assert np.array_equal(around.view(np.uint8), np.full(around.size, poison, nptype(t)).view(np.uint8))
+    y = dec(np.ascontiguousarray(body[:, :hidden]), t)
+    assert np.isnan(y[4]).all()
+    keep = [i for i in range(rows) if i != 4]
+    xq, gq, bq = dec(xe, t)[keep], dec(ge, t), dec(be, t)
+    if layer:
+        check_norm(y[keep], O.layernorm(xq, gq, bq, 1e-6), bq, t)
+    else:
+        check_norm(y[keep], O.rmsnorm(xq, gq, 1e-6), None, t)
