@@ -2062,7 +2062,8 @@ inline int64_t general_blocks(const GemmDesc& d) {
 // workgroups on a CU, and no more than there are stages. bf16 N,N 128x500x500,
 // with 1 / 2 / 4 groups: 8 members (128 workgroups) 16.6 / 10.7 / 8.5 us, 28
 // (448) 19.4 / 14.3 / 16.9, 64 (1024) 26.7 / 27.2 / 32.4. int8 (whose M-
-// contiguous staging spills with 4 groups) N,T 999x199x611: 11.4 / 8.6 / 13.9.
+// contiguous staging spills 63 VGPRs with 4 groups, which are not built for it)
+// N,T 999x199x611: 11.4 / 8.6 / 13.9.
 template <class Op>
 int general_groups(const GemmDesc& d) {
   const int64_t blocks = general_blocks(d);
@@ -2331,9 +2332,9 @@ hipError_t run(const GemmDesc& d, hipStream_t s) {
     constexpr int VE = 16 / Op::kElemBytes;
     const int groups = p.probe ? 1 : general_groups<Op>(*g);
     if ((g->ta ? g->k : g->m) < VE || (g->tb ? g->n : g->k) < VE) go(gemm_general<Op, OUT, 1, true>, 1);
-    else if (groups == 4) go(gemm_general<Op, OUT, 4, false>, 4);
     else if (groups == 2) go(gemm_general<Op, OUT, 2, false>, 2);
-    else go(gemm_general<Op, OUT, 1, false>, 1);
+    else if (groups == 1) go(gemm_general<Op, OUT, 1, false>, 1);
+    else if constexpr (VE < 16) go(gemm_general<Op, OUT, 4, false>, 4);   // int8 takes at most 2
   }
   return hipGetLastError();
 }

@@ -36,7 +36,6 @@ struct SParams {
   int64_t lda, ldb, ldc;
   int64_t sa, sb, sc;
   int m, n, k;
-  int ta, tb;
   int tiles_m;
   float alpha, beta;
   grxCycleSlot* probe;
@@ -116,7 +115,7 @@ void sgemm_mfma(SParams p) {
   float* C = p.c + bz * p.sc;
   const bool interior = row0 + MT <= p.m && col0 + MT <= p.n;
 
-  // Staging: an operand stage is MT x 16 elements read along its storage's
+  // Staging: an operand stage is MT x kK elements read along its storage's
   // contiguous dimension (op(A): i for N, k for T; op(B): k for N, j for T)
   // in groups of 4 consecutive elements; thread t handles groups
   // t + 256*q. Element (cont, other) of a group maps to LDS [kk][i or j].
@@ -535,7 +534,6 @@ hipError_t launch_sgemm(const SgemmDesc& d, hipStream_t s) {
   p.lda = d.lda; p.ldb = d.ldb; p.ldc = d.ldc;
   p.sa = d.stride_a; p.sb = d.stride_b; p.sc = d.stride_c;
   p.m = d.m; p.n = d.n; p.k = d.k;
-  p.ta = d.ta; p.tb = d.tb;
   p.alpha = d.alpha; p.beta = d.beta;
   p.probe = d.probe;
   if (d.batch > 65535) return hipErrorInvalidValue;
