@@ -304,9 +304,14 @@ __device__ __forceinline__ void attend_tile(const AParams& p, const LanePos& l, 
         mx1 = fmaxf(mx1, s[1][r]);
       }
       const float mx = half_swap_max(fmaxf(mx0, mx1));
-      const bool raise = fmaf(mx, p.c, -m_run) > 8.0f;
+      // (>=: where 8 is lost in the rounding, equal maxima may still differ by
+      // half an ulp, which scaled_max looks at. The difference as one fma
+      // schedules the whole tile worse, 2 % at D = 64.)
+      const bool raise = mx * p.c >= m_run + 8.0f;
       if (__builtin_amdgcn_ballot_w64(raise)) {
-        const float m_new = raise ? scaled_max<T>(mx, p.c) : m_run;
+        float top = scaled_max<T>(mx, p.c);
+        asm("" : "+v"(top));   // a select, not a branch of its own
+        const float m_new = raise ? top : m_run;
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
         m_run = m_new;
         l_run *= alpha;

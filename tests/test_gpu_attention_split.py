@@ -93,3 +93,28 @@ def test_attention_masked_keys(dnn, D, H, S, t, fill, causal):
             assert np.isnan(o[0, h, :lo]).all()
         assert np.isfinite(o[0, h, lo:]).all(), name
         assert normwise_rel_err(o[0, h, lo:], ref[lo:]) <= 1e-2, name
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_attention_masked_group_maxima(dnn, causal):
+    """Scores -1.5 * 2^35 and 4096 more (one ulp): scaled, both round to one
+    float, which the first lies below and the second exceeds by 482 (the
+    exponent of an overflowing weight). The group of the tiles 1 and 5, which
+    hold them, must still add 0."""
+    c = np.float32(0.125) * np.float32(1.4426950408889634)
+    s = np.float32([-1.5 * 2.0 ** 35, -1.5 * 2.0 ** 35 + 4096])
+    m, exact = (s * c).astype(np.float64), s.astype(np.float64) * np.float64(c)
+    assert m[0] == m[1] and exact[0] < m[0] and exact[1] > m[1] + 140
+    H, S, D = 6, 500, 64
+    r = np.random.default_rng(8)
+    q = r.standard_normal((1, H, S, D)).astype(np.float32)
+    k = r.standard_normal((1, H, S, D)).astype(np.float32)
+    q[..., :2] = 1.0
+    for tile, low in ((1, 0.0), (5, 4096.0)):
+        k[:, :, 64 * tile:64 * tile + 64] = 0.0
+        k[:, :, 64 * tile:64 * tile + 64, 0] = -1.5 * 2.0 ** 35
+        k[:, :, 64 * tile:64 * tile + 64, 1] = low
+    o, qq, kq, v = run_attention(dnn, BF16, 1, H, S, D, causal, seed=8, q=q, k=k)
+    assert np.isfinite(o).all()
+    for h in range(H):
+        assert normwise_rel_err(o[0, h], O.attention_head(qq[0, h], kq[0, h], v[0, h], causal, D ** -0.5)) <= 1e-2, h
