@@ -53,6 +53,8 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdio>
+#include <cstdlib>
 
 namespace grxk {
 namespace {
@@ -587,8 +589,6 @@ __global__ __launch_bounds__(64 * kNW, 1) void attn_fwd(AParams p) {
 // ceil(S/(32*QW)) CUs instead of S/64 on ceil(S/256). NS LDS stages of KS
 // tiles: with two, a step's loads are issued one step ahead; with one (the
 // tiles of a step fill LDS) the next step's loads wait for this one's reads.
-// A wave alone in its group (QW = 1) reads only what it loaded and needs no
-// barrier.
 template <AttnType T, int D, int QW, int NS>
 __global__ __launch_bounds__(64 * kNW, 1) void attn_split(AParams p) {
   using IO = AIo<T>;
@@ -599,7 +599,7 @@ __global__ __launch_bounds__(64 * kNW, 1) void attn_split(AParams p) {
   constexpr int kPitch = D + 4;                    // floats per row of a wave's O in LDS
   constexpr int kStageBytes = NS * KS * 2 * kTile * 16;
   constexpr int kMergeBytes = kNW * 32 * kPitch * 4;
-  static_assert(NS == 1 || NS == 2, "stages");
+  static_assert((QW == 2 || QW == 4) && (NS == 1 || NS == 2), "query blocks, stages");
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kStageBytes > kMergeBytes ? kStageBytes : kMergeBytes];
   __shared__ float ml[kNW][2][32];                 // running maximum and sum per query
 
@@ -652,7 +652,7 @@ __global__ __launch_bounds__(64 * kNW, 1) void attn_split(AParams p) {
   };
   auto landed = [&]() __attribute__((always_inline)) {
     wait_vmem_all();
-    if constexpr (QW > 1) __syncthreads();
+    __syncthreads();
   };
 
   load(0, 0);
@@ -682,8 +682,7 @@ __global__ __launch_bounds__(64 * kNW, 1) void attn_split(AParams p) {
       attend_tile<T, D>(p, lp, (const i32x4*)tile_at(st, 0), tile_at(st, 1), kv0, wq0, qf, o_acc, m_run, l_run);
     if (NS == 1 && s + 1 < steps) {
       // every read of this step's tiles is done before the next one's land
-      if constexpr (QW > 1) __syncthreads();
-      else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __syncthreads();
       load(s + 1, 0);
     }
     if (s + 1 < steps) landed();
@@ -741,14 +740,18 @@ __global__ __launch_bounds__(64 * kNW, 1) void attn_split(AParams p) {
   }
 }
 
-// One workgroup per CU, a multiple of 8 (one share per XCD), no more than
-// the items need.
-int64_t workgroups(int B, int H, int S) {
+// CUs of the current device, a multiple of 8 (one share per XCD).
+int compute_units() {
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess)
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  return std::max(8, cus / 8 * 8);
+}
+
+// One workgroup per CU, no more than the items need.
+int64_t workgroups(int cus, int B, int H, int S) {
   const int64_t qtiles = (S + kBQ - 1) / kBQ;
-  int64_t wgs = (cus / 8) * 8;
+  int64_t wgs = cus;
   const int64_t per_xcd_items = ((int64_t)B * H + 7) / 8 * qtiles;
   if (wgs / 8 > per_xcd_items) wgs = 8 * per_xcd_items;
   if (wgs < 8) wgs = 8;
@@ -772,12 +775,12 @@ int heads_per_block(int64_t hx, int qtiles, int nwg, bool causal) {
 // attn_fwd, whichever is modelled fastest (us; the constants fit bf16 times of
 // 64 to 4000 keys on 4 to 256 heads). A CU runs one tile (or step of KS tiles)
 // at a time, so a launch takes the steps of its busiest CU: the heaviest item
-// while there are at most 256, the average CU's share beyond, plus a start and
-// an end per item, which the persistent kernel hides. us, attn_fwd / QW 4 / QW
-// 2: B2 H16 S1000 D64 24.0 / 16.9 / 21.9; B1 H8 S2048 D64 38.6 / 24.0 / 16.5
+// while there is at most one per CU, the average CU's share beyond, plus a start
+// and an end per item, which the persistent kernel hides. us, attn_fwd / QW 4 /
+// QW 2: B2 H16 S1000 D64 24.0 / 16.9 / 21.9; B1 H8 S2048 D64 38.6 / 24.0 / 16.5
 // and D128 49.9 / 33.6 / 27.0; B1 H24 S218 D128 12.3 / 9.8 / 8.5; B4 H16
 // S1024 D64 23.5 / 24.1 / 36.2 and D128 36.5 / 43.1 / 63.6.
-int split_blocks(int64_t heads, int S, int D, bool causal) {
+int split_blocks(int cus, int64_t heads, int S, int D, bool causal) {
   const double start = D == 64 ? 3.5 : 4.0;
   // Mean tiles of an item of `queries` over the heaviest item's.
   auto share = [&](int queries) {
@@ -785,26 +788,42 @@ int split_blocks(int64_t heads, int S, int D, bool causal) {
     return causal ? (n + 1.0) / (2.0 * n) : 1.0;
   };
   const double tiles = (S + kBK - 1) / kBK;
-  // attn_fwd: the items of one XCD's heads over its 32 workgroups
-  const double items8 = (double)((heads + 7) / 8) * ((S + kBQ - 1) / kBQ) / 32.0;
+  // attn_fwd: the items of one XCD's heads over its workgroups
+  const double items8 = (double)((heads + 7) / 8) * ((S + kBQ - 1) / kBQ) / (cus / 8);
   const double rounds = causal ? std::max(1.0, 1.1 * items8 * share(kBQ)) : std::ceil(items8);
   double best = 0.95 * (start + (D == 64 ? 1.25 : 1.8) * tiles * rounds);
   int qw = 0;
   for (int w = 4; w >= 2; w /= 2) {
-    const double items = (double)heads * ((S + 32 * w - 1) / (32 * w)) / 256.0;   // per CU
+    const double items = (double)heads * ((S + 32 * w - 1) / (32 * w)) / cus;   // per CU
     const double steps = std::ceil(tiles * w / kNW) * (items > 1.0 ? share(32 * w) : 1.0);
     const double step = D == 64 ? (w == 4 ? 1.55 : 1.65) : (w == 4 ? 2.2 : 3.0);
     double t;
-    if (D == 64 && w == 4)   // two workgroups share a CU
-      t = start + std::max(1.0, items) * (steps * step + 0.6);
-    else
+    if (D == 64 && w == 4) {
+      // Two workgroups share a CU. Items of one size leave some CUs a whole one
+      // more than others, of which sharing hides a fifth (90 heads of 317 keys
+      // 12.2 us, attn_fwd 10.5).
+      const double busiest = causal || items <= 1.0 ? items : std::max(items, 0.82 * std::ceil(items));
+      t = start + std::max(1.0, busiest) * (steps * step + 0.6);
+      // Beside one round of attn_fwd the heaviest item counts: it shares its CU
+      // with a light one, and a head's items lie on several XCDs where heads are
+      // no multiple of 8 (causal, 110 heads of 307 keys 10.8 us, attn_fwd 10.3).
+      if (causal && items > 1.0 && items8 <= 1.0 && heads % 8)
+        t = std::max(t, start + std::ceil(tiles * w / kNW) * step + 1.4);
+    } else {
       t = std::ceil(items) * (start + (D == 128 && w == 2 ? 0.8 : 0.2) + steps * step);
+    }
     if (t < best) {
       best = t;
       qw = w;
     }
   }
   return qw;
+}
+
+// GRXDNN_LOG set (and not "0"): one line on stderr per attention call.
+bool log_launches() {
+  const char* v = std::getenv("GRXDNN_LOG");
+  return v && *v && !(v[0] == '0' && v[1] == 0);
 }
 
 template <AttnType T, int D>
@@ -830,17 +849,23 @@ hipError_t run(const AttnDesc& d, hipStream_t s) {
   if (span >= (1ll << 31)) return hipErrorNotSupported;
   // item indices are 32-bit in the kernel
   if ((int64_t)d.B * d.H * p.qtiles > 0x7fffffff) return hipErrorInvalidValue;
+  const int cus = compute_units();
   // (a cycle probe's slots are counted for attn_fwd)
-  const int qw = d.probe ? 0 : split_blocks((int64_t)d.B * d.H, d.S, D, p.causal);
+  int qw = d.probe ? 0 : split_blocks(cus, (int64_t)d.B * d.H, d.S, D, p.causal);
   const int64_t items = qw ? (int64_t)p.heads * ((d.S + 32 * qw - 1) / (32 * qw)) : 0;
-  if (qw && items <= max_workgroups(64 * kNW)) {
+  if (items > max_workgroups(64 * kNW)) qw = 0;
+  if (log_launches())
+    std::fprintf(stderr, "grxdnn: attention %s b=%d h=%d s=%d d=%d causal=%d kernel=%s\n",
+                 T == AttnType::BF16 ? "bf16" : "f16", d.B, d.H, d.S, D, (int)p.causal,
+                 qw == 4 ? "split4" : qw == 2 ? "split2" : "fwd");
+  if (qw) {
     p.qtiles = (d.S + 32 * qw - 1) / (32 * qw);
     const dim3 grid((unsigned)items);
     if (qw == 4) hipLaunchKernelGGL((attn_split<T, D, 4, 2>), grid, dim3(64 * kNW), 0, s, p);
     else hipLaunchKernelGGL((attn_split<T, D, 2, D == 64 ? 2 : 1>), grid, dim3(64 * kNW), 0, s, p);
     return hipGetLastError();
   }
-  const int64_t wgs = workgroups(d.B, d.H, d.S);
+  const int64_t wgs = workgroups(cus, d.B, d.H, d.S);
   p.hb = heads_per_block((p.heads + 7) / 8, p.qtiles, (int)(wgs / 8), p.causal);
   hipLaunchKernelGGL((attn_fwd<T, D>), dim3((unsigned)wgs), dim3(64 * kNW), 0, s, p);
   return hipGetLastError();
@@ -848,7 +873,7 @@ hipError_t run(const AttnDesc& d, hipStream_t s) {
 
 }  // namespace
 
-int64_t attention_probe_slots(int B, int H, int S) { return workgroups(B, H, S) * kNW; }
+int64_t attention_probe_slots(int B, int H, int S) { return workgroups(compute_units(), B, H, S) * kNW; }
 
 hipError_t launch_attention(AttnType t, const AttnDesc& d, hipStream_t s) {
   if (t == AttnType::BF16) {

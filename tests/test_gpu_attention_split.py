@@ -2,13 +2,15 @@
 workgroups split the keys over two or four groups of waves (attn_split), and
 causal launches whose heads form one block of the persistent kernel's item
 order. Every head against the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import grxcp_amd as g
 import oracle as O
-from helpers import normwise_rel_err
-from test_gpu_dnn import run_attention
+from helpers import normwise_rel_err, say, to_dev
+from test_gpu_dnn import dec, enc, run_attention
 
 pytestmark = pytest.mark.gpu
 BF16, F16 = g.GRX_R_16BF, g.GRX_R_16F
@@ -118,3 +120,34 @@ def test_attention_masked_group_maxima(dnn, causal):
     assert np.isfinite(o).all()
     for h in range(H):
         assert normwise_rel_err(o[0, h], O.attention_head(qq[0, h], kq[0, h], v[0, h], causal, D ** -0.5)) <= 1e-2, h
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("t", [BF16, F16])
+@pytest.mark.parametrize("H,S,D,kernel", [(24, 517, 64, "split2"), (24, 517, 128, "split2"), (40, 390, 64, "split4"),
+                                          (40, 390, 128, "split4"), (200, 300, 64, "fwd"), (200, 300, 128, "fwd"),
+                                          (90, 317, 64, "fwd")])   # 270 items of 128 queries on 256 CUs
+def test_attention_kernel_choice(dnn, capfd, monkeypatch, H, S, D, kernel, t, causal):
+    """Each kernel by its name in the log, on a packed [S, 3, H, D] buffer with
+    partial key and query tiles. Heads are copies of five, which must agree."""
+    r = np.random.default_rng(S + D)
+    x = enc(r.standard_normal((S, 3, 5, D)).astype(np.float32), t).reshape(S, 3, 5, D)
+    qkv = np.ascontiguousarray(x[:, :, np.arange(H) % 5])
+    dx, do = to_dev(qkv), g.DeviceBuffer(2 * S * H * D)
+    xd = g.TensorDesc(t, [1, H, S, D], [3 * S * H * D, D, 3 * H * D, 1])
+    od = g.TensorDesc(t, [1, H, S, D], [S * H * D, D, H * D, 1])
+    at = [ctypes.c_void_p(dx.p.value + 2 * H * D * i) for i in range(3)]
+    say(f"attention t={t} H={H} S={S} D={D} causal={causal}, packed: {kernel}")
+    capfd.readouterr()
+    monkeypatch.setenv("GRXDNN_LOG", "1")
+    s = dnn.attention(g.AttnDesc(causal, D ** -0.5), xd, at[0], xd, at[1], xd, at[2], od, do.p)
+    monkeypatch.delenv("GRXDNN_LOG")
+    assert s == g.SUCCESS, g.STATUS[s]
+    g.synchronize()
+    log = [l for l in capfd.readouterr().err.splitlines() if l.startswith("grxdnn: attention ")]
+    assert len(log) == 1 and log[0].endswith(f"kernel={kernel}"), log
+    o = dec(do.download(np.uint16, S * H * D), t).reshape(S, H, D)
+    for h in range(5):
+        q, k, v = (dec(np.ascontiguousarray(x[:, i, h]), t).reshape(S, D) for i in range(3))
+        assert normwise_rel_err(o[:, h], O.attention_head(q, k, v, causal, D ** -0.5)) <= 1e-2, h
+        assert np.array_equal(o[:, h::5], np.repeat(o[:, h:h + 1], len(range(h, H, 5)), 1)), h
