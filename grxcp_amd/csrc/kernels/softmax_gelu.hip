@@ -13,8 +13,10 @@
 // three passes (max, sum, write) re-reading x.
 // GELU: one 16-byte chunk per thread, over the tensor as one array when its
 // rows are contiguous, else row by row; erf or tanh form in fp32, rounded once.
-// Rows off 16-byte boundaries (an odd length or pitch) run the same kernels on
-// chunks at element alignment with a partial last chunk (AL = false).
+// Rows off 16-byte boundaries (an odd length or pitch) run the same kernels
+// (AL = false) on chunks that lie on memory's 16-byte boundaries, the first and
+// last of a row partial (RowChunks); where a kernel has no room for one chunk
+// more, and for contiguous GELU, at element alignment with a partial end.
 
 #include "../launch.h"
 #include "device_common.h"

@@ -230,7 +230,12 @@ grxblasStatus_t grxblasSetKernelPath(const char* path);
 
 /* Per-wave cycle records (ref grxblas.h:240-242). With a slot array attached,
  * the next Sgemm/GemmEx calls record one grxCycleSlot per wave. capacity must
- * cover grxblasCycleSlotsNeeded for the call. NULL turns recording off. */
+ * cover grxblasCycleSlotsNeeded for the call. NULL turns recording off.
+ * A recorded call runs a kernel of the launch that its slots are counted for,
+ * which need not be the one that the call runs without a probe: GemmEx in one
+ * pass over K (no slices, no K groups, no few-column kernel), Sgemm on 128x128
+ * or 64x64 tiles without K groups, Sgemv with 256 rows or one column per
+ * workgroup. */
 grxblasStatus_t grxblasSetCycleProbe(grxblasHandle_t handle,
                                      grxCycleSlot* slots, int capacity);
 int             grxblasCycleSlotsNeeded(grxblasHandle_t handle, int m, int n);

@@ -159,7 +159,10 @@ grxdnnStatus_t grxdnnAttentionForward(grxdnnHandle_t handle,
  * workgroup * waves per workgroup + wave; s_memtime at entry and exit, core
  * = XCD << 16 | CU id); capacity must cover
  * grxdnnAttentionCycleSlotsNeeded for the call's B, H and S, else the call
- * returns INVALID_VALUE before any device work. NULL turns recording off. */
+ * returns INVALID_VALUE before any device work. NULL turns recording off.
+ * A recorded call always runs the persistent kernel that the slots are counted
+ * for, also where the call alone would split its keys over workgroups of fewer
+ * queries. */
 grxdnnStatus_t grxdnnSetCycleProbe(grxdnnHandle_t handle, grxCycleSlot* slots,
                                    int capacity);
 int            grxdnnAttentionCycleSlotsNeeded(grxdnnHandle_t handle, int batch,
