@@ -1771,6 +1771,7 @@ template <class Op>
 bool skinny_wanted(const GemmDesc& d) {
   const int64_t kbytes = (int64_t)d.k * Op::kElemBytes;
   if (d.batch != 1 || d.probe || d.n > 64 || kbytes < 4 * kFastKBytes || !tn_operands_ready<Op>(d)) return false;
+  if (d.m > 16 * max_workgroups(512)) return false;   // more workgroups than one launch takes
   if (d.m > 4096)
     return kbytes <= (d.n <= 16 || (d.n <= 32 && d.m <= 8192) ? 8192 : 4096) &&
            (d.n <= 32 || d.m * kbytes <= (64ll << 20));

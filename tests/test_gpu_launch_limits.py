@@ -65,3 +65,27 @@ def test_softmax_many_unaligned_rows(gpu, dnn):
         got = dec(x.download(np.uint16, hidden, offset=2 * hidden * i), BF16)
         assert np.all(np.abs(got - ref) <= 2.0 ** -8 * np.abs(ref)), i
     x.close()
+
+
+def test_gemm_many_rows_of_few_columns(gpu, blas):
+    """2^27 + 16 rows of one column, 16 rows to a 512-thread workgroup of
+    gemm_skinny: the wider tiles' kernel."""
+    m, n, k = (1 << 27) + 16, 1, 256
+    a = big_buffer(gpu, 2 * m * k)
+    c = g.DeviceBuffer(4 * m)
+    r = np.random.default_rng(2)
+    rows = enc(r.standard_normal((64, k)).astype(np.float32), BF16).reshape(64, k)
+    b = enc(r.standard_normal((1, k)).astype(np.float32), BF16).reshape(1, k)
+    at = (0, m // 2, m - 64)
+    for i in at:
+        a.upload(rows, offset=2 * k * i)
+    db = to_dev(b)
+    say("GemmEx of 2^27 + 16 rows and one column")
+    s = blas.gemm_ex(1, 0, m, n, k, 1.0, a.p, BF16, k, db.p, BF16, k, 0.0, c.p, g.GRX_R_32F, m)
+    assert s == g.SUCCESS, g.STATUS[s]
+    g.synchronize()
+    ref = dec(rows, BF16).reshape(64, k).astype(np.float64) @ dec(b, BF16).reshape(k).astype(np.float64)
+    for i in at:
+        assert normwise_rel_err(c.download(np.float32, 64, offset=4 * i), ref) <= 1e-5, i
+    c.close()
+    a.close()
