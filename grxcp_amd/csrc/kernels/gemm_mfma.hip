@@ -1761,23 +1761,31 @@ bool tn_ready(const GemmDesc& d) {
 // columns 28 KB (2048 rows 19 / 19, at 64 KB 47 / 39), 16 columns 24 KB (256
 // rows 16 / 15, at 128 KB 73 / 38), 32 columns 16 KB (1024 rows 15.9 / 16, at
 // 32 KB 26 / 16), 64 columns 10 KB (17 / 17, at 16 KB 21 / 16). With more rows
-// memory bounds both: 4096 x 16, K of 32 KB 32 / 38, of 64 KB 55 / 67, of 80
-// KB 67 / 63; 3584 x 8 of 80 KB 55 / 59; 4096 x 32 of 32 KB 35 / 39, of 40 KB
-// 44 / 38. Past 4096 rows a CU has several workgroups, each reading B again:
-// 16384 x 16 x 4096 27.5 / 38.1, 8192 x 20 x 4096 19.6 / 20 (of 8192 34.1 /
-// 35.6), 12288 x 32 of 4 KB 19 / 20, of 8 KB none gained; 16384 x 40 x 1024
-// 10.7 / 12.4, but 16384 x 64 x 4096 42.7 / 41.1.
+// memory bounds both, and the two meet later: 3 columns nowhere (2576 rows 28
+// KB to 128 KB), 8 columns past 48 KB (3136 rows of 48 KB 1.07 times as fast,
+// of 65 KB 42.1 / 43.5 at 3008), 16 past 40 KB (3648 rows of 40 KB 33.1 / 33.2,
+// of 48 KB 40.5 / 38.2), 32 past 22 KB (3584 rows of 20 KB 1.3 times as fast, of
+// 24 KB 23.9 / 21.7, of 28 KB 29.2 / 24.2). (K a power of two is the tiles' bad
+// case: 4096 rows, 16 columns of 64 KB 1.25 times as fast here; the lines are
+// drawn where no other K loses.) Past 4096 rows a CU has several workgroups,
+// each reading B again: 16384 x 16 x 4096 27.5 / 38.1, 8192 x 20 x 4096 19.6 /
+// 20 (of 8192 34.1 / 35.6), 9024 x 32 of 4 KB 1.25 times as fast, 16000 x 32 of 4
+// KB 21.2 / 19.0; 16384 x 40 x 1024 10.7 / 12.4, but 16384 x 64 x 4096 42.7 /
+// 41.1.
 template <class Op>
 bool skinny_wanted(const GemmDesc& d) {
   const int64_t kbytes = (int64_t)d.k * Op::kElemBytes;
   if (d.batch != 1 || d.probe || d.n > 64 || kbytes < 4 * kFastKBytes || !tn_operands_ready<Op>(d)) return false;
   if (d.m > 16 * max_workgroups(512)) return false;   // more workgroups than one launch takes
-  if (d.m > 4096)
-    return kbytes <= (d.n <= 16 || (d.n <= 32 && d.m <= 8192) ? 8192 : 4096) &&
-           (d.n <= 32 || d.m * kbytes <= (64ll << 20));
-  if (d.n <= 8) return d.m > 2560 || kbytes <= (28 << 10);
-  if (d.n <= 16) return kbytes <= (d.m > 3072 ? 64 << 10 : 24 << 10);
-  if (d.n <= 32) return kbytes <= (d.m > 3072 ? 32 << 10 : 16 << 10);
+  if (d.m > 4096) {
+    if (d.n <= 16) return kbytes <= 8192;
+    if (d.n <= 32) return kbytes <= (d.m <= 8192 ? 8192 : 4096) && d.m <= 12288;
+    return kbytes <= 4096 && d.m * kbytes <= (64ll << 20);
+  }
+  if (d.n <= 4) return d.m > 2560 || kbytes <= (28 << 10);
+  if (d.n <= 8) return kbytes <= (d.m > 2560 ? 48 << 10 : 28 << 10);
+  if (d.n <= 16) return kbytes <= (d.m > 3072 ? 40 << 10 : 24 << 10);
+  if (d.n <= 32) return kbytes <= (d.m > 3072 ? 22 << 10 : 16 << 10);
   return kbytes <= (10 << 10);
 }
 

@@ -52,8 +52,9 @@ def test_skinny_limits(blas, capfd):
         assert [p["kernel"] for p in plans] != ["skinny"], (m, n, k, pad)
 
 
-@pytest.mark.parametrize("m,n,kmax", [(16, 8, 14336), (2576, 3, 0), (128, 16, 12288), (3088, 32, 16384),
-                                      (128, 17, 8192), (64, 33, 5120), (4096, 64, 5120)])
+@pytest.mark.parametrize("m,n,kmax", [(16, 8, 14336), (2576, 3, 0), (128, 16, 12288), (3088, 32, 11264),
+                                      (128, 17, 8192), (64, 33, 5120), (4096, 64, 5120),
+                                      (2576, 8, 24576), (3088, 9, 20480), (8208, 17, 2048), (12304, 16, 4096)])
 def test_skinny_k_bound(blas, capfd, m, n, kmax):
     """K of the longest that one workgroup takes runs on gemm_skinny, K one
     16-byte chunk longer on the 128x128 tiles and their K slices (kmax 0: no
