@@ -45,8 +45,8 @@ struct NParams {
   int64_t rows;
   int rows_per_wg;     // norm_block: adjacent rows per workgroup
   int hidden;
-  int align_mask;      // unaligned rows: RowChunks
   float eps;
+  int align_mask;      // unaligned rows: RowChunks
 };
 
 // One row per NT-thread workgroup, NQ 16-byte chunks per thread (chunk

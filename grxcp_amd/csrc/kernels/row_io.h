@@ -93,9 +93,9 @@ struct RowChunks {
     if constexpr (!AL) head = (int)((uintptr_t)row / (16 / V)) & align_mask;
   }
   __device__ __forceinline__ int first(int c) const { return c * V - (AL ? 0 : head); }
-  __device__ __forceinline__ bool any(int c) const { return first(c) < hidden; }
+  __device__ __forceinline__ bool any(int c) const { return AL ? c < hidden / V : first(c) < hidden; }
   __device__ __forceinline__ bool whole(int c) const {
-    return (AL || first(c) >= 0) && first(c) + V <= hidden;
+    return AL ? any(c) : first(c) >= 0 && first(c) + V <= hidden;
   }
   __device__ __forceinline__ bool has(int c, int e) const {
     return AL || (first(c) + e >= 0 && first(c) + e < hidden);
